@@ -105,7 +105,8 @@ size_t xnq_qtensor_device_bytes(const xnq_qtensor* qt);
  * route is chosen from m and the shape: a wavefront-per-row matvec for small
  * m (Q4_K / Q6_K up to 4 rows, up to 2 for K >= 4096 and 2048 < N <= K),
  * the small-batch int8 MFMA kernel up to 64 rows, the
- * tiled int8 MFMA kernel for prefill-sized m.  Validates what xn validates:
+ * tiled int8 MFMA kernel for prefill-sized m; the other dtypes the matvec up
+ * to 8 rows and the f16 MFMA kernels above).  Validates what xn validates:
  * mkn against the weight shape (repack.rs:203-215) and m*k == lhs length is
  * the caller's contract.  Stream ordered; allocates its activation scratch
  * stream-ordered (hipMallocAsync). */

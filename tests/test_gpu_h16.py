@@ -1,0 +1,136 @@
+"""The f16 matrix-core kernels (k_h16.hip) against the CPU oracle: every type
+they take, at the edges of their tiles (32 and 64 rows, 32 and 256 columns),
+of their K stages (128 and 256, with the remainders of K), and of the rule
+that chooses between them; tiny (f16 subnormal) scales; infinities and NaN in
+the activations against the matvec kernels; the slabs of matmul_t_noalloc.
+
+The kernels' block sums are exact integers and their sums over K are 32-bit,
+so the outputs are held to 32-bit sums of K / 32 terms: relative L2 2e-6
+(the oracle itself sums in f32)."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+Q4_0, Q4_1, Q5_0, Q5_1, Q8_0, Q2K, Q3K, Q5K = 2, 3, 6, 7, 8, 10, 11, 13
+BLOCK32 = [Q4_0, Q4_1, Q5_0, Q5_1, Q8_0]
+SUPER = [Q2K, Q3K, Q5K]
+
+
+def upload(blocks, n, k, dt, dev):
+    from xn_amd import GgmlDType, QTensor
+
+    return QTensor.from_gguf_bytes(blocks, (n, k), GgmlDType(dt), dev)
+
+
+def run(qt, x, m, k, n, dev):
+    dst = torch.full((m, n), float("nan"), dtype=torch.float32, device=dev)
+    qt.matmul_t((m, k, n), torch.from_numpy(x).to(dev), dst)
+    return dst.cpu().numpy()
+
+
+def check(orc, dev, dt, m, k, n, seed, wscale=0.02, xscale=1.0):
+    rng = np.random.default_rng(seed)
+    blocks = orc.from_float(dt, (rng.normal(0, wscale, (n, k))).astype(np.float32))
+    x = (rng.normal(0, xscale, (m, k))).astype(np.float32)
+    got = run(upload(blocks, n, k, dt, dev), x, m, k, n, dev).astype(np.float64)
+    want = orc.matmul(dt, x, blocks, n).astype(np.float64)
+    assert np.isfinite(got).all()
+    rel = np.linalg.norm(got - want) / np.linalg.norm(want)
+    assert rel < 2e-6, f"dt={dt} m={m} k={k} n={n}: rel {rel}"
+
+
+# K-split kernel: one and two row tiles, ragged columns, K stages cut short
+@pytest.mark.parametrize("dt", BLOCK32)
+@pytest.mark.parametrize("m,k,n", [(9, 64, 31), (32, 192, 33), (33, 1088, 65), (17, 4160, 96), (64, 2048, 8200)])
+def test_block_types_ksplit(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 100 + dt + m)
+
+
+@pytest.mark.parametrize("dt", [Q4_0, Q8_0])
+@pytest.mark.parametrize("k", [32, 96, 160, 1056])
+def test_odd_block_counts(orc, dev, dt, k):
+    check(orc, dev, dt, 37, k, 40, 200 + dt + k)
+
+
+@pytest.mark.parametrize("dt", SUPER)
+@pytest.mark.parametrize("m,k,n", [(9, 256, 31), (32, 512, 33), (33, 2304, 65), (17, 4352, 96), (65, 2048, 8200)])
+def test_super_types_ksplit(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 300 + dt + m)
+
+
+# the 256 x 64 tile: full and ragged last tiles, K past its 16-step output sums
+@pytest.mark.parametrize("dt,m,k,n", [(dt, 640, 64, 3841) for dt in BLOCK32] + [(dt, 577, 2112, 4096) for dt in BLOCK32]
+                         + [(dt, 600, 4160, 3840) for dt in (Q4_0, Q5_1, Q8_0)])
+def test_block_types_tile(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 400 + dt + m)
+
+
+@pytest.mark.parametrize("dt", [Q4_0, Q8_0])
+def test_block_types_tile_odd_blocks(orc, dev, dt):
+    check(orc, dev, dt, 600, 1056, 3842, 500 + dt)
+
+
+@pytest.mark.parametrize("dt", SUPER)
+@pytest.mark.parametrize("m,k,n", [(512, 256, 3585), (449, 1280, 4096)])
+def test_super_types_tile(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 600 + dt + m)
+
+
+# block scales in the f16 subnormal range, on either side
+@pytest.mark.parametrize("dt", BLOCK32 + SUPER)
+@pytest.mark.parametrize("wscale,xscale", [(2e-5, 1.0), (0.02, 2e-4)])
+def test_subnormal_scales(orc, dev, dt, wscale, xscale):
+    check(orc, dev, dt, 40, 1024, 64, 700 + dt, wscale, xscale)
+
+
+@pytest.mark.parametrize("dt", [Q4_0, Q4_1, Q8_0, Q2K, Q5K])
+@pytest.mark.parametrize("m,n", [(40, 64), (600, 3840)])
+def test_nonfinite_rows(orc, dev, dt, m, n):
+    """An infinity, a NaN and an overflowing scale in an activation row reach
+    the same outputs as on the matvec kernels, and no other row."""
+    from xn_amd.quantized import set_route
+
+    rng = np.random.default_rng(800 + dt)
+    k = 512
+    blocks = orc.from_float(dt, rng.normal(0, 0.02, (n, k)).astype(np.float32))
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    x[3, 7], x[5, 300], x[20, 40] = np.inf, np.nan, 1e9
+    x[8] = 0.0
+    qt = upload(blocks, n, k, dt, dev)
+    got = run(qt, x, m, k, n, dev)
+    try:
+        set_route(1)
+        want = run(qt, x, m, k, n, dev)
+    finally:
+        set_route(0)
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    assert (got[8] == 0).all()
+    ok = np.isfinite(want).all(axis=1)
+    err = np.linalg.norm(got[ok].astype(np.float64) - want[ok]) / np.linalg.norm(want[ok].astype(np.float64))
+    assert err < 2e-6
+
+
+@pytest.mark.parametrize("dt", [Q8_0, Q5K])
+def test_noalloc_slabs(orc, dev, dt):
+    """More rows than the static scratch holds with their f16 copy, but not
+    without it: the same outputs as with a workspace."""
+    from xn_amd import XnqError
+
+    k, n, m = 4096, 64, 8000
+    rng = np.random.default_rng(900 + dt)
+    blocks = orc.from_float(dt, rng.normal(0, 0.02, (n, k)).astype(np.float32))
+    qt = upload(blocks, n, k, dt, dev)
+    assert qt.matmul_t_workspace_size(m) > (64 << 20)
+    x = torch.randn((m, k), generator=torch.Generator(device=dev).manual_seed(5), device=dev)
+    want = torch.empty((m, n), device=dev)
+    got = torch.full((m, n), float("nan"), device=dev)
+    qt.matmul_t((m, k, n), x, want)
+    qt.matmul_t_noalloc((m, k, n), x, got)
+    assert ((got - want).norm() / want.norm()).item() < 1e-6
+    # past the rows whose images alone fill it, it refuses as before
+    big = torch.zeros((16000, k), device=dev)
+    with pytest.raises(XnqError, match="scratch"):
+        qt.matmul_t_noalloc((16000, k, n), big, torch.empty((16000, n), device=dev))

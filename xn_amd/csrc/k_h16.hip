@@ -1,0 +1,1030 @@
+// Quantized matmul on the f16 matrix cores for the weight types the int8
+// digit kernels do not take (Q8_0, Q4_0, Q4_1, Q5_0, Q5_1; Q2K, Q3K, Q5K),
+// from a few rows up to prefill sizes.
+//
+// Exactness.  Every level of these formats times its integer sub-block scale
+// (Q5K: 6-bit scale x 5-bit level <= 1953) and every 8-bit activation level
+// is a whole number that f16 holds exactly, their products are exact, and
+// the sum of one block (|I| < 2^24) is exact in the f32 accumulator: the
+// matrix core returns the same integer block dot the reference forms
+// (k_quants.rs:287-304, 419-440, 513-544, 677-691, 899-948, 1071-1152,
+// 1524-1605), as a float and without a conversion.
+//
+// Scales.  The 32-element types scale every 32 K: y += (d_w d_a) I.  Both
+// scales are f16, so their outer product over a 32 x 32 tile is one more
+// MFMA with a single non-zero K slot, exact in f32, and the epilogue is one
+// fma per output element (with the product formed on the vector units it is
+// two, and with an int8 contraction three).  The K types scale every 256 K:
+// y += d_a (d_w I1 - dmin I2), where I2 = sum_g m_g bsum_g is one K = 16 MFMA
+// of the sub-block mins by the 16 block sums, exact for the same reason.
+//
+// Operands.  Weight columns are MFMA operand A (expanded to f16 in registers
+// right before use: a nibble or byte b becomes 0x6400 | b = 1024 + b, then one
+// packed add or fma), activation rows operand B, read as f16 in MFMA order
+// from the activation image (H16Img).  Lane (column or row l & 31, half
+// l >> 5) holds elements 16 half .. 16 half + 15 of each 32-element chunk, as
+// two K = 16 steps.
+//
+// Summation.  Long chains of f32 additions are split so that the rounding
+// error stays at the level of the matvec kernels' lane tree: four blocks,
+// then four stages, then the rest, then (wavefronts that split K) a tree.
+#include <type_traits>
+
+#include "xnq_device.h"
+#include "xnq_internal.h"
+
+namespace xnq {
+
+namespace {
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+typedef float f16v __attribute__((ext_vector_type(16)));
+
+constexpr int kThreads = 512, kWaves = 8;
+
+// What one 32-column stage of a weight type is: CH chunks of 32 K, SEG bytes
+// of the q plane per column, fetched with LDS DMA as P pieces of PB bytes (16
+// where blocks are 8-byte aligned, else 4) in NI instructions of a wavefront,
+// column after column.  The scales of the plane types (Q8_0, Q4_0) take one
+// more instruction.
+template <int DT>
+struct HT {
+    static constexpr bool kK = is_kquant(DT);
+    static constexpr int kCH = kK ? 8 : 4;
+    static constexpr int kSeg = DT == XNQ_Q8_0 ? 128 : DT == XNQ_Q4_0 ? 64 : kK ? (int)raw_stride(DT) : 4 * (int)raw_stride(DT);
+    static constexpr int kPB = DT == XNQ_Q2K || DT == XNQ_Q4_1 ? 4 : 16;
+    static constexpr int kP = kSeg / kPB;
+    static constexpr int kNI = (32 * kP + 63) / 64;
+    static constexpr bool kPlaneD = DT == XNQ_Q8_0 || DT == XNQ_Q4_0;  // d in a plane of its own
+    static constexpr bool kMin32 = DT == XNQ_Q4_1 || DT == XNQ_Q5_1;
+    static constexpr bool kMinK = DT == XNQ_Q2K || DT == XNQ_Q5K;
+    static constexpr int kSlot = kNI * 64 * kPB + (kPlaneD ? 256 : 0);  // one stage in LDS
+    static constexpr int kND = kNI + (kPlaneD ? 1 : 0);                 // DMA instructions of a stage
+    static constexpr int kDl = kK ? 256 : 0;  // d_w, dmin by column (K types)
+};
+
+// LDS offset of piece p of column c in a stage.  Powers of two are swizzled so
+// that the eight lanes of one read phase fall in different banks; the odd and
+// 6-piece strides spread by themselves.
+template <int DT>
+__device__ __forceinline__ uint32_t piece_off(uint32_t c, uint32_t p) {
+    if (DT == XNQ_Q8_0) return (c * 8 + (p ^ ((c >> 1) & 7))) * 16;
+    if (DT == XNQ_Q4_0) return (c * 4 + (p ^ ((c >> 2) & 3))) * 16;
+    return (c * HT<DT>::kP + p) * HT<DT>::kPB;
+}
+
+// 1024 + byte for bytes (0, 1) and (2, 3) of x
+__device__ __forceinline__ h2 magic01(uint32_t x) {
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, x, 0x04010400u));
+}
+__device__ __forceinline__ h2 magic23(uint32_t x) {
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u));
+}
+__device__ __forceinline__ h2 splat2(float v) {
+    const _Float16 h = (_Float16)v;
+    return h2{h, h};
+}
+
+// Per-lane plane offsets of the DMA of a 32-column tile, without the stage's
+// own offset.
+template <int DT>
+struct WOff {
+    uint32_t row[HT<DT>::kNI], in[HT<DT>::kNI];  // column's row offset, offset in the stage's segment
+    uint32_t d;
+};
+
+template <int DT>
+__device__ __forceinline__ void weight_offsets(WOff<DT>& o, const WView& w, uint32_t col0, uint32_t lane) {
+    using T = HT<DT>;
+#pragma unroll
+    for (int i = 0; i < T::kNI; i++) {
+        const uint32_t idx = min(i * 64 + lane, 32u * T::kP - 1), c = idx / T::kP;
+        uint32_t p = idx % T::kP;
+        if (DT == XNQ_Q8_0) p ^= (c >> 1) & 7;
+        if (DT == XNQ_Q4_0) p ^= (c >> 2) & 3;
+        o.row[i] = min(col0 + c, w.n - 1) * w.q_row;
+        o.in[i] = p * T::kPB;
+    }
+    o.d = T::kPlaneD ? min(col0 + (lane >> 1), w.n - 1) * w.d_row + (lane & 1) * 4 : 0u;
+}
+
+// DMA of stage st into the LDS slot at byte address `to`.  A stage past the end of the row
+// (K not a multiple of 128) re-reads the row's last piece; its scales are zeroed.
+template <int DT, bool DV>
+__device__ __forceinline__ void issue_weights(const WOff<DT>& o, const WView& w, uint32_t st, uint32_t to) {
+    using T = HT<DT>;
+#pragma unroll
+    for (int i = 0; i < T::kNI; i++) {
+        uint32_t off = st * T::kSeg + o.in[i];
+        if (!T::kK && !(T::kPlaneD && DV)) off = min(off, w.q_row - T::kPB);
+        if (T::kPB == 16) dma16(w.q, o.row[i] + off, to + i * 1024);
+        else dma4(w.q, o.row[i] + off, to + i * 256);
+    }
+    if (T::kPlaneD && DV) dma4(w.d, o.d + st * 8, to + T::kNI * 1024);
+}
+
+// 16 bytes of LDS at a 4-byte aligned address
+__device__ __forceinline__ uint4 lds16(const uint8_t* p) {
+    const uint32_t* q = reinterpret_cast<const uint32_t*>(p);
+    return make_uint4(q[0], q[1], q[2], q[3]);
+}
+
+// bits 0-3 of t, one to bit 4 of each byte (t < 16: the product has no carries)
+__device__ __forceinline__ uint32_t spread_bit4(uint32_t t) { return (__umul24(t, 0x00204081u) & 0x01010101u) << 4; }
+
+// The bytes of chunk j that a lane expands: its 16 levels' low bits, and high
+// bits where the type has them apart.
+struct Bytes {
+    uint4 v, w;
+};
+
+// `slot` is the stage in LDS, c the column, h the lane half.
+template <int DT>
+__device__ __forceinline__ void read_chunk(Bytes& r, const uint8_t* slot, uint32_t c, int j, uint32_t h) {
+    const uint8_t* col = slot + c * HT<DT>::kSeg;  // (block types)
+    if constexpr (DT == XNQ_Q8_0) {
+        r.v = *reinterpret_cast<const uint4*>(slot + piece_off<DT>(c, 2 * j + h));
+    } else if constexpr (DT == XNQ_Q4_0) {
+        r.v = *reinterpret_cast<const uint4*>(slot + piece_off<DT>(c, j));
+    } else if constexpr (DT == XNQ_Q4_1) {
+        r.v = lds16(col + j * 20 + 4);
+    } else if constexpr (DT == XNQ_Q5_0 || DT == XNQ_Q5_1) {
+        r.v = lds16(col + j * 24 + 8);
+        r.w.x = *reinterpret_cast<const uint32_t*>(col + j * 24 + 4);
+    } else if constexpr (DT == XNQ_Q5K) {
+        // chunk j = 2i + s: nibble s of qs bytes 32i .. 32i+31, fifth bit j of qh
+        r.v = *reinterpret_cast<const uint4*>(col + 48 + 32 * (j >> 1) + 16 * h);
+        r.w = *reinterpret_cast<const uint4*>(col + 16 + 16 * h);
+    } else {
+        // Q2K, Q3K: chunk j = 4h' + t: bits 2t of qs bytes 32h' .. 32h'+31; Q3K's third bit j of hmask
+        r.v = lds16(col + (DT == XNQ_Q2K ? 16 : 32) + 32 * (j >> 2) + 16 * h);
+        if (DT == XNQ_Q3K) r.w = lds16(col + 16 * h);
+    }
+}
+
+// Operand A of chunk j: the lane's 16 levels (times the sub-block scale, K
+// types) as two K = 16 steps; hd the block header words a K type needs.
+template <int DT>
+__device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const uint4& hd, h8* a) {
+    const uint32_t v[4] = {r.v.x, r.v.y, r.v.z, r.v.w}, w[4] = {r.w.x, r.w.y, r.w.z, r.w.w};
+    uint32_t x[4];  // four levels a dword, as bytes
+    float bias = 0.f, sc = 0.f;
+    if constexpr (DT == XNQ_Q8_0) {
+#pragma unroll
+        for (int d = 0; d < 4; d++) x[d] = v[d] ^ 0x80808080u;
+        bias = -1152.f;
+    } else if constexpr (!HT<DT>::kK) {
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            x[d] = (v[d] >> (4 * h)) & 0x0F0F0F0Fu;
+            if (DT == XNQ_Q5_0 || DT == XNQ_Q5_1) x[d] |= spread_bit4((w[0] >> (16 * h + 4 * d)) & 15u);
+        }
+        bias = DT == XNQ_Q4_0 ? -1032.f : DT == XNQ_Q5_0 ? -1040.f : -1024.f;
+    } else if constexpr (DT == XNQ_Q5K) {
+#pragma unroll
+        for (int d = 0; d < 4; d++)
+            x[d] = ((v[d] >> (4 * (j & 1))) & 0x0F0F0F0Fu) | ((j >= 4 ? w[d] >> (j - 4) : w[d] << (4 - j)) & 0x10101010u);
+        const Q4KScales q = q4k_scales(hd.y, hd.z, hd.w);
+        sc = (float)(((j < 4 ? q.sc_lo : q.sc_hi) >> (8 * (j & 3))) & 0xffu);
+    } else {
+#pragma unroll
+        for (int d = 0; d < 4; d++) x[d] = (v[d] >> (2 * (j & 3))) & 0x03030303u;
+        if constexpr (DT == XNQ_Q3K) {  // the lane's 16 elements are sub-block 2j + h
+#pragma unroll
+            for (int d = 0; d < 4; d++) x[d] |= (j >= 2 ? w[d] >> (j - 2) : w[d] << (2 - j)) & 0x04040404u;
+            sc = (float)(q3k_scale(hd.x, hd.y, hd.z, (int)(2 * j + h)) - 32);
+        } else {
+            const uint32_t hw = (j >> 1) == 0 ? hd.x : (j >> 1) == 1 ? hd.y : (j >> 1) == 2 ? hd.z : hd.w;
+            sc = (float)((hw >> (8 * (2 * (j & 1) + h))) & 15u);
+        }
+    }
+    h2 q[8];
+#pragma unroll
+    for (int d = 0; d < 4; d++) {
+        q[2 * d] = magic01(x[d]);
+        q[2 * d + 1] = magic23(x[d]);
+    }
+    if constexpr (!HT<DT>::kK) {
+        const h2 b = splat2(bias);
+#pragma unroll
+        for (int d = 0; d < 8; d++) q[d] = q[d] + b;
+    } else if constexpr (DT == XNQ_Q3K) {
+        const h2 b = splat2(-1028.f), s = splat2(sc);
+#pragma unroll
+        for (int d = 0; d < 8; d++) q[d] = (q[d] + b) * s;
+    } else {
+        // (1024 + q) sc - 1024 sc, exact: 1024 sc is a 6-bit number times 2^10
+        const h2 s = splat2(sc), b = splat2(-1024.f * sc);
+#pragma unroll
+        for (int d = 0; d < 8; d++) q[d] = __builtin_elementwise_fma(q[d], s, b);
+    }
+    a[0] = h8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+    a[1] = h8{q[4].x, q[4].y, q[5].x, q[5].y, q[6].x, q[6].y, q[7].x, q[7].y};
+}
+
+__device__ __forceinline__ f16v mfma16(h8 a, h8 b, f16v c) {
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+// the K = 8 step takes half the operand registers: for the rank-1 products
+__device__ __forceinline__ f16v mfma8(uint2 a, uint2 b) {
+    return __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), f16v{}, 0, 0, 0);
+}
+__device__ __forceinline__ h8 as_h8(uint4 v) { return __builtin_bit_cast(h8, v); }
+
+// What a stage needs of its weights beside the levels.
+template <int DT>
+struct Scales {
+    uint4 hd;                            // K types: the block header's words
+    uint2 d[HT<DT>::kK ? 1 : 4];      // 32-element types: operand of the scale product, chunk j
+    uint2 m[HT<DT>::kMin32 ? 4 : 1];  // and of the min product (the chunk's K slot only)
+    uint4 mn;                            // K types: min-term operand
+};
+
+// Reads a stage's scales from its slot; K types also leave d_w and dmin by
+// column at dl (a wavefront's own LDS: its operations stay in order).
+template <int DT, bool DV>
+__device__ __forceinline__ void read_scales(Scales<DT>& S, const WView& w, const uint8_t* slot, uint8_t* dl,
+                                            uint32_t col0, uint32_t lane, uint32_t st, uint32_t nch) {
+    using T = HT<DT>;
+    const uint32_t c = lane & 31, h = lane >> 5;
+    const uint8_t* col = slot + c * T::kSeg;
+    if constexpr (T::kK) {
+        uint32_t dd;
+        if constexpr (DT == XNQ_Q5K) {
+            S.hd = *reinterpret_cast<const uint4*>(col);
+            dd = S.hd.x;
+        } else if constexpr (DT == XNQ_Q2K) {
+            S.hd = lds16(col);  // the 16 scale / min bytes
+            dd = *reinterpret_cast<const uint32_t*>(col + 80);
+        } else {
+            S.hd = lds16(col + 96);
+            dd = S.hd.w & 0xffffu;
+        }
+        reinterpret_cast<float*>(dl)[lane] = f16_bits_to_f32(h ? dd >> 16 : dd & 0xffffu);  // [dw 32][dmin 32]
+        if constexpr (T::kMinK) {
+            // mins of sub-blocks (16 elements each) 8h .. 8h + 7
+            h8 mv;
+            if constexpr (DT == XNQ_Q5K) {
+                const Q4KScales q = q4k_scales(S.hd.y, S.hd.z, S.hd.w);
+                const uint32_t mw = h ? q.m_hi : q.m_lo;
+#pragma unroll
+                for (int t = 0; t < 8; t++) mv[t] = (_Float16)(float)((mw >> (8 * (t >> 1))) & 0xffu);
+            } else {
+                const uint32_t b0 = h ? S.hd.z : S.hd.x, b1 = h ? S.hd.w : S.hd.y;
+#pragma unroll
+                for (int t = 0; t < 8; t++) mv[t] = (_Float16)(float)(((t < 4 ? b0 : b1) >> (8 * (t & 3) + 4)) & 15u);
+            }
+            S.mn = __builtin_bit_cast(uint4, mv);
+        }
+    } else {
+        uint32_t dv[4];
+        if constexpr (T::kPlaneD && DV) {
+            const uint2 v = *reinterpret_cast<const uint2*>(slot + T::kNI * 1024 + c * 8);
+            dv[0] = v.x & 0xffffu; dv[1] = v.x >> 16; dv[2] = v.y & 0xffffu; dv[3] = v.y >> 16;
+        } else if constexpr (T::kPlaneD) {
+            const uint16_t* dp = reinterpret_cast<const uint16_t*>(w.d + min(col0 + c, w.n - 1) * w.d_row);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t v = dp[min(st * 4 + j, nch - 1)];
+                dv[j] = st * 4 + j < nch ? v : 0u;
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t f = *reinterpret_cast<const uint32_t*>(col + j * (int)raw_stride(DT));
+                const bool live = st * 4 + j < nch;
+                dv[j] = live ? f & 0xffffu : 0u;
+                if constexpr (T::kMin32) {
+                    const uint32_t mv = live && h == 0 ? f >> 16 : 0u;
+                    const uint32_t v = j & 1 ? mv << 16 : mv;
+                    S.m[j] = j < 2 ? make_uint2(v, 0) : make_uint2(0, v);
+                }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) S.d[j] = make_uint2(h == 0 ? dv[j] : 0u, 0);
+    }
+}
+
+// One 32 x 32 unit (a chunk of a 32-element type by a row tile): the matrix
+// products, and their fold into the running sum t.
+template <int DT>
+struct Unit {
+    f16v I, sc, p;
+};
+template <int DT>
+__device__ __forceinline__ void unit_mma(Unit<DT>& u, const h8* a, const Scales<DT>& S, int j, const uint4* b,
+                                         const uint2& bd, const uint2& bs) {
+    u.I = mfma16(a[0], as_h8(b[0]), f16v{});
+    u.sc = mfma8(S.d[j], bd);
+    u.I = mfma16(a[1], as_h8(b[1]), u.I);
+    if constexpr (HT<DT>::kMin32) u.p = mfma8(S.m[j], bs);
+}
+template <int DT>
+__device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t) {
+#pragma unroll
+    for (int e = 0; e < 16; e++) {
+        if constexpr (HT<DT>::kMin32) {
+            // per block, as the reference's vec_dot: the min and main terms cancel
+            const float v = fmaf(u.I[e], u.sc[e], u.p[e]);
+            t[e] = first ? v : t[e] + v;
+        } else {
+            t[e] = first ? u.I[e] * u.sc[e] : fmaf(u.I[e], u.sc[e], t[e]);
+        }
+    }
+}
+
+// A super-block's sums I (and the min sums) of a 32 x 32 tile into the output.
+template <int DT>
+__device__ __forceinline__ void super_unit(const f16v& I, const Scales<DT>& S, const uint4& bs, float da, const float* dw,
+                                           const float* dm, f16v& out) {
+    if constexpr (HT<DT>::kMinK) {
+        const f16v I2 = mfma16(as_h8(S.mn), as_h8(bs), f16v{});
+#pragma unroll
+        for (int e = 0; e < 16; e++) out[e] = fmaf(da, fmaf(dw[e], I[e], -(dm[e] * I2[e])), out[e]);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; e++) out[e] = fmaf(da * dw[e], I[e], out[e]);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Few rows, or few tiles: a workgroup owns 32 weight columns and 32 TM rows,
+// and its eight wavefronts split K, so that a weight of a few thousand columns
+// still puts two wavefronts on every SIMD.  Each wavefront streams its share of
+// the weights through its own LDS ring (LDS DMA in whole cache lines, two
+// stages ahead) and its share of the activation image straight into registers
+// (a stage ahead); there is no barrier until the eight partial tiles are added,
+// in a tree, through LDS.
+// ---------------------------------------------------------------------------
+template <int DT, int TM, bool DV>
+__global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
+                                                              uint32_t n_tiles, float* __restrict__ y) {
+    using T = HT<DT>;
+    constexpr int kU = T::kCH * TM;       // (chunk, tile) units of a stage
+    constexpr int kPD = kU < 8 ? kU : 8;  // units whose operand B is in flight
+    constexpr int kSlots = 3, kWaveLds = kSlots * T::kSlot + T::kDl;
+    constexpr int kRed = kWaves * TM * 4 * 64 * 16;
+    constexpr int kLds = kWaves * kWaveLds > kRed ? kWaves * kWaveLds : kRed;
+    static_assert(kLds <= 160 * 1024, "LDS budget");
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t total = m_tiles * n_tiles, per = (total + 7) / 8;
+    const uint32_t wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // one XCD: consecutive items, one column tile
+    if (wi >= total) return;
+    const uint32_t mt = wi % m_tiles, nt = wi / m_tiles;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col0 = nt * 32, nch = w.k / 32;
+    const uint32_t nst = (nch + T::kCH - 1) / T::kCH, wst = (nst + kWaves - 1) / kWaves;
+    const uint32_t s0 = min(wave * wst, nst), s1 = min(s0 + wst, nst);
+    uint8_t* wl = lds + wave * kWaveLds;
+    uint8_t* dl = wl + kSlots * T::kSlot;
+    const uint32_t wbase = (uint32_t)(uintptr_t)lds + wave * kWaveLds;
+    const H16Img& H = a.H;
+    const uint32_t lrow = lane & 31, g = lane >> 5;
+
+    // lanes of rows past m read the last row again (their outputs are dropped)
+    uint32_t rt[TM], bl[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) {
+        rt[i] = min(mt * TM + i, H.rts - 1);
+        bl[i] = g * 32 + min(lrow, m - 1 - rt[i] * 32);
+    }
+
+    f16v out[TM], mid[TM];
+#pragma unroll
+    for (int i = 0; i < TM; i++) out[i] = mid[i] = f16v{};
+
+    if (s0 < s1) {
+        WOff<DT> wo;
+        weight_offsets<DT>(wo, w, col0, lane);
+        uint4 b[kPD][2];
+        uint2 bd[T::kK ? 1 : kPD];
+        float da[TM];    // K types: d_a of the stage's super-block
+        uint4 bs[TM];    // and min-term operand
+        uint2 bs32[TM];  // Q4_1, Q5_1: min-term operand of the stage
+        auto load_unit = [&](uint32_t st, int u, int slot) {
+            const int j = u / TM, i = u % TM;
+            const uint32_t c = min(st * T::kCH + j, nch - 1);
+            const uint8_t* p = a.h16 + ((size_t)rt[i] * nch + c) * 2048 + bl[i] * 16;
+            b[slot][0] = *reinterpret_cast<const uint4*>(p);
+            b[slot][1] = *reinterpret_cast<const uint4*>(p + 1024);
+            if constexpr (!T::kK)
+                bd[slot] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt[i] * nch + c) * 512 + lane * 8);
+        };
+        auto load_scales = [&](uint32_t st) {
+#pragma unroll
+            for (int i = 0; i < TM; i++) {
+                if constexpr (T::kK) {
+                    da[i] = reinterpret_cast<const float*>(a.h16 + H.d_off + ((size_t)rt[i] * nst + st) * 128)[lrow];
+                    if constexpr (T::kMinK)
+                        bs[i] = *reinterpret_cast<const uint4*>(a.h16 + H.s_off + ((size_t)rt[i] * nst + st) * 1024 + lane * 16);
+                } else if constexpr (T::kMin32) {
+                    bs32[i] = *reinterpret_cast<const uint2*>(a.h16 + H.s_off + ((size_t)rt[i] * nst + st) * 512 + lane * 8);
+                }
+            }
+        };
+        issue_weights<DT, DV>(wo, w, s0, wbase);
+        issue_weights<DT, DV>(wo, w, min(s0 + 1, s1 - 1), wbase + T::kSlot);
+#pragma unroll
+        for (int u = 0; u < kPD; u++) load_unit(s0, u, u);
+        load_scales(s0);
+        asm volatile("" ::: "memory");
+        issue_weights<DT, DV>(wo, w, min(s0 + 2, s1 - 1), wbase + 2 * T::kSlot);
+        uint32_t slot = 0;
+        for (uint32_t s = s0; s < s1; s++) {
+            const uint32_t sn = min(s + 1, s1 - 1);
+            // the DMA of stages s + 1 and s + 2 is younger than this stage's
+            wait_vm<2 * ((T::kPlaneD && !DV) ? T::kNI : T::kND)>();
+            const uint8_t* ws = wl + slot * T::kSlot;
+            Scales<DT> S;
+            read_scales<DT, DV>(S, w, ws, dl, col0, lane, s, nch);
+            if constexpr (T::kK) {
+                f16v I[TM];
+#pragma unroll
+                for (int j = 0; j < T::kCH; j++) {
+                    h8 A[2];
+                    Bytes by;
+                    read_chunk<DT>(by, ws, lrow, j, g);
+                    expand<DT>(by, j, g, S.hd, A);
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+                        const int u = j * TM + i;
+                        I[i] = mfma16(A[0], as_h8(b[u % kPD][0]), j == 0 ? f16v{} : I[i]);
+                        I[i] = mfma16(A[1], as_h8(b[u % kPD][1]), I[i]);
+                        if (u + kPD < kU) load_unit(s, u + kPD, u % kPD);
+                        else load_unit(sn, u + kPD - kU, u % kPD);
+                    }
+                }
+                float dw[16], dm[16];
+                const float* dp = reinterpret_cast<const float*>(dl) + 4 * g;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    dw[e] = dp[8 * (e >> 2) + (e & 3)];
+                    if (T::kMinK) dm[e] = dp[32 + 8 * (e >> 2) + (e & 3)];
+                }
+#pragma unroll
+                for (int i = 0; i < TM; i++) super_unit<DT>(I[i], S, bs[i], da[i], dw, dm, out[i]);
+            } else {
+                f16v t[TM];
+#pragma unroll
+                for (int j = 0; j < T::kCH; j++) {
+                    h8 A[2];
+                    Bytes by;
+                    read_chunk<DT>(by, ws, lrow, j, g);
+                    expand<DT>(by, j, g, S.hd, A);
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+                        const int u = j * TM + i;
+                        Unit<DT> un;
+                        unit_mma<DT>(un, A, S, j, b[u % kPD], bd[u % kPD], bs32[i]);
+                        unit_add<DT>(un, j == 0, t[i]);
+                        if (u + kPD < kU) load_unit(s, u + kPD, u % kPD);
+                        else load_unit(sn, u + kPD - kU, u % kPD);
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < TM; i++) {
+#pragma unroll
+                    for (int e = 0; e < 16; e++) mid[i][e] += t[i][e];
+                }
+                if ((s & 3) == 3) {
+#pragma unroll
+                    for (int i = 0; i < TM; i++) {
+#pragma unroll
+                        for (int e = 0; e < 16; e++) out[i][e] += mid[i][e];
+                        mid[i] = f16v{};
+                    }
+                }
+            }
+            load_scales(sn);
+            // this stage's slot is read; fetch stage s + 3 into it
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue_weights<DT, DV>(wo, w, min(s + 3, s1 - 1), wbase + slot * T::kSlot);
+            slot = slot == 2 ? 0 : slot + 1;
+        }
+        wait_vm<0>();  // no DMA may land in the reduction below
+    }
+    // partial tiles to LDS ([wave][tile, quad][lane] float4), then one quad of
+    // one tile per wavefront, summed over the eight in a tree
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            float4 v;
+            v.x = out[i][4 * q] + mid[i][4 * q];
+            v.y = out[i][4 * q + 1] + mid[i][4 * q + 1];
+            v.z = out[i][4 * q + 2] + mid[i][4 * q + 2];
+            v.w = out[i][4 * q + 3] + mid[i][4 * q + 3];
+            reinterpret_cast<float4*>(lds)[(wave * (TM * 4) + i * 4 + q) * 64 + lane] = v;
+        }
+    __syncthreads();
+    for (uint32_t iq = wave; iq < TM * 4; iq += kWaves) {
+        float4 p[8];
+#pragma unroll
+        for (int v = 0; v < 8; v++) p[v] = reinterpret_cast<const float4*>(lds)[(v * (TM * 4) + iq) * 64 + lane];
+#pragma unroll
+        for (int d = 1; d < 8; d *= 2)
+#pragma unroll
+            for (int v = 0; v < 8; v += 2 * d) {
+                p[v].x += p[v + d].x;
+                p[v].y += p[v + d].y;
+                p[v].z += p[v + d].z;
+                p[v].w += p[v + d].w;
+            }
+        const uint32_t row = (mt * TM + (iq >> 2)) * 32 + lrow, n = col0 + 8 * (iq & 3) + 4 * g;
+        if (row >= m) continue;
+        float* yr = y + (size_t)row * w.n + n;
+        if ((w.n & 3) == 0 && n + 3 < w.n) {
+            *reinterpret_cast<float4*>(yr) = p[0];
+        } else {
+            if (n < w.n) yr[0] = p[0].x;
+            if (n + 1 < w.n) yr[1] = p[0].y;
+            if (n + 2 < w.n) yr[2] = p[0].z;
+            if (n + 3 < w.n) yr[3] = p[0].w;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Prefill sizes: a workgroup of eight wavefronts owns 256 weight columns and
+// 64 rows; wavefront w owns columns 32w .. 32w+31 and every row, so each
+// weight is expanded once per workgroup, and the activation tile is shared
+// through LDS.  K advances four chunks (128) a step.  All data moves by LDS
+// DMA: the activation tile (1 KiB pieces, shared) into a three-slot ring two
+// steps ahead, each wavefront's own weights into two slots one stage ahead.
+// One barrier per step publishes the shared pieces; each wavefront waits for
+// its own DMA by exact count.
+//
+// K types (this kernel): 32 x 32 tiles, a stage is a super-block and two steps.
+// ---------------------------------------------------------------------------
+template <int DT>
+struct TLay {
+    using T = HT<DT>;
+    static constexpr int kBSlot = 2 * 4 * 2048 + (T::kK ? 0 : 2 * 2048 + (T::kMin32 ? 2 * 512 : 0));  // quants (, scales, sums)
+    static constexpr int kSc = 2 * 4 * 2048, kMs = kSc + 2 * 2048;  // offsets in a slot
+    static constexpr int kSb = T::kK ? 2 * 128 + (T::kMinK ? 2 * 1024 : 0) : 0;  // a super-block's d_a, sums
+    static constexpr int kOffW = 3 * kBSlot;
+    static constexpr int kOffSb = kOffW + kWaves * 2 * T::kSlot;
+    static constexpr int kOffDl = kOffSb + 2 * kSb;
+    static constexpr int kLds = kOffDl + kWaves * T::kDl;
+    static_assert(kLds <= 160 * 1024, "LDS budget");
+    // DMA instructions of every wavefront: per step, and per super-block
+    static constexpr int kNB = 2 + (T::kK ? 0 : 1) + (T::kMin32 ? 1 : 0);
+    static constexpr int kNSb = T::kK ? 1 + (T::kMinK ? 1 : 0) : 0;
+};
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
+                                                                  uint32_t n_tiles, float* __restrict__ y) {
+    using T = HT<DT>;
+    using Y = TLay<DT>;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t total = m_tiles * n_tiles, per = (total + 7) / 8;
+    const uint32_t wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // one XCD: consecutive items, which share columns
+    if (wi >= total) return;
+    const uint32_t mt = wi % m_tiles, nt = wi / m_tiles;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lrow = lane & 31, g = lane >> 5;
+    const uint32_t col0 = nt * 256 + wave * 32, nch = w.k / 32, nsb = nch / 8, nstep = nch / 4;
+    const uint32_t lbase = (uint32_t)(uintptr_t)lds;
+    const H16Img& H = a.H;
+    const uint32_t rt0 = mt * 2, rt1 = min(mt * 2 + 1, H.rts - 1);
+
+    // ---- DMA: step q's activation tile, a super-block's scales and sums, its weights ----
+    auto issue_b = [&](uint32_t q, uint32_t slot) {
+        const uint32_t c = min(q, nstep - 1) * 4 + (wave >> 1), to = lbase + slot * Y::kBSlot + wave * 1024;
+        dma16(a.h16 + ((size_t)rt0 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to);
+        dma16(a.h16 + ((size_t)rt1 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to + 8192);
+    };
+    const uint8_t* const d0 = a.h16 + H.d_off + (size_t)rt0 * nsb * 128;
+    auto issue_sb = [&](uint32_t sb, uint32_t slot) {
+        const uint32_t sc = min(sb, nsb - 1), to = lbase + Y::kOffSb + slot * Y::kSb;
+        dma4(d0 + sc * 128, (g ? (rt1 - rt0) * nsb * 128 : 0u) + lrow * 4, to);
+        if constexpr (T::kMinK)  // of row tile wave & 1 (repeats are the same bytes)
+            dma16(a.h16 + H.s_off + ((size_t)(wave & 1 ? rt1 : rt0) * nsb + sc) * 1024, lane * 16,
+                  to + 256 + (wave & 1) * 1024);
+    };
+    WOff<DT> wo;
+    weight_offsets<DT>(wo, w, col0, lane);
+    const uint32_t wls = Y::kOffW + wave * (2 * T::kSlot);
+    auto issue_w = [&](uint32_t sb, uint32_t slot) {
+        issue_weights<DT, true>(wo, w, min(sb, nsb - 1), lbase + wls + slot * T::kSlot);
+    };
+
+    f16v out[2], I[2];
+#pragma unroll
+    for (int i = 0; i < 2; i++) out[i] = f16v{};
+    issue_b(0, 0);
+    issue_sb(0, 0);
+    issue_w(0, 0);
+    issue_b(1, 1);
+    uint32_t slot = 0, free_slot = 2;
+    Scales<DT> S;
+    uint8_t* dl = lds + Y::kOffDl + wave * T::kDl;
+    for (uint32_t sb = 0; sb < nsb; sb++) {
+        const uint8_t* ws = lds + wls + (sb & 1) * T::kSlot;
+        const uint8_t* sbp = lds + Y::kOffSb + (sb & 1) * Y::kSb;
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            // this step has landed, and every wavefront is past the previous one.  Younger
+            // than its DMA: at the first step the next step's tile, at the second also the
+            // next super-block's pieces
+            if (p == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB) : "memory");
+            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB + Y::kNSb + T::kND) : "memory");
+            issue_b(2 * sb + p + 2, free_slot);
+            if (p == 0) {
+                issue_sb(sb + 1, (sb + 1) & 1);
+                issue_w(sb + 1, (sb + 1) & 1);
+                read_scales<DT, true>(S, w, ws, dl, col0, lane, sb, nch);
+            }
+            const uint8_t* bs = lds + slot * Y::kBSlot + lane * 16;
+#pragma unroll
+            for (int jj = 0; jj < 4; jj++) {
+                const int j = 4 * p + jj;
+                h8 A[2];
+                Bytes by;
+                read_chunk<DT>(by, ws, lrow, j, g);
+                expand<DT>(by, j, g, S.hd, A);
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    const uint4 b0 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048);
+                    const uint4 b1 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048 + 1024);
+                    I[i] = mfma16(A[0], as_h8(b0), j == 0 ? f16v{} : I[i]);
+                    I[i] = mfma16(A[1], as_h8(b1), I[i]);
+                }
+            }
+            free_slot = slot;
+            slot = slot == 2 ? 0 : slot + 1;
+        }
+        float dw[16], dm[16];
+        const float* dp = reinterpret_cast<const float*>(dl) + 4 * g;
+#pragma unroll
+        for (int e = 0; e < 16; e++) {
+            dw[e] = dp[8 * (e >> 2) + (e & 3)];
+            if (T::kMinK) dm[e] = dp[32 + 8 * (e >> 2) + (e & 3)];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            const float da = reinterpret_cast<const float*>(sbp)[i * 32 + lrow];
+            uint4 ms = make_uint4(0, 0, 0, 0);
+            if constexpr (T::kMinK) ms = *reinterpret_cast<const uint4*>(sbp + 256 + i * 1024 + lane * 16);
+            super_unit<DT>(I[i], S, ms, da, dw, dm, out[i]);
+        }
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup's LDS
+    const uint32_t nb0 = col0 + 4 * g;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        const uint32_t row = mt * 64 + i * 32 + lrow;
+        if (row >= m) continue;
+        float* yr = y + (size_t)row * w.n;
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const uint32_t n = nb0 + 8 * q;
+            if (n + 3 < w.n && (w.n & 3) == 0) {
+                *reinterpret_cast<float4*>(yr + n) =
+                    make_float4(out[i][4 * q], out[i][4 * q + 1], out[i][4 * q + 2], out[i][4 * q + 3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    if (n + e < w.n) yr[n + e] = out[i][4 * q + e];
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The 32-element types at prefill sizes, on 16 x 16 tiles: one K = 32 product
+// is one chunk, and the four sums and four scales of a tile take 8 registers,
+// so the products of one row group are in flight while the previous one's are
+// folded, within the 256 registers that two wavefronts per SIMD leave each.
+// (On 32 x 32 tiles the same pipeline needs 96 registers and spills, and a
+// spill's reload waits for every DMA in flight.)
+// ---------------------------------------------------------------------------
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+template <int DT>
+__device__ __forceinline__ void read_chunk8(uint2& v, uint32_t& qh, const uint8_t* slot, uint32_t c, int j, uint32_t kg) {
+    const uint8_t* col = slot + c * HT<DT>::kSeg;
+    const uint32_t o = 8 * (kg & 1);
+    if constexpr (DT == XNQ_Q8_0) {
+        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, 2 * j + (kg >> 1)) + o);
+    } else if constexpr (DT == XNQ_Q4_0) {
+        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, j) + o);
+    } else if constexpr (DT == XNQ_Q4_1) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(col + j * 20 + 4 + o);
+        v = make_uint2(p[0], p[1]);
+    } else {
+        v = *reinterpret_cast<const uint2*>(col + j * 24 + 8 + o);
+        qh = *reinterpret_cast<const uint32_t*>(col + j * 24 + 4);
+    }
+}
+
+template <int DT>
+__device__ __forceinline__ h8 expand8(const uint2& v, uint32_t qh, uint32_t kg) {
+    const uint32_t d[2] = {v.x, v.y};
+    h2 q[4];
+    const h2 b = splat2(DT == XNQ_Q8_0 ? -1152.f : DT == XNQ_Q4_0 ? -1032.f : DT == XNQ_Q5_0 ? -1040.f : -1024.f);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        uint32_t x;
+        if constexpr (DT == XNQ_Q8_0) {
+            x = d[i] ^ 0x80808080u;
+        } else {
+            x = (d[i] >> (4 * (kg >> 1))) & 0x0F0F0F0Fu;
+            if (DT == XNQ_Q5_0 || DT == XNQ_Q5_1) x |= spread_bit4((qh >> (8 * kg + 4 * i)) & 15u);
+        }
+        q[2 * i] = magic01(x) + b;
+        q[2 * i + 1] = magic23(x) + b;
+    }
+    return h8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+__device__ __forceinline__ f4v mfma16x16x32(h8 a, h8 b) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f4v{}, 0, 0, 0);
+}
+__device__ __forceinline__ f4v mfma16x16x16(uint2 a, uint2 b) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), f4v{}, 0, 0, 0);
+}
+
+template <int DT, bool DV>
+__global__ __launch_bounds__(kThreads) void h16_block_tile_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
+                                                                  uint32_t n_tiles, float* __restrict__ y) {
+    using T = HT<DT>;
+    using Y = TLay<DT>;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t total = m_tiles * n_tiles, per = (total + 7) / 8;
+    const uint32_t wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // one XCD: consecutive items, which share columns
+    if (wi >= total) return;
+    const uint32_t mt = wi % m_tiles, nt = wi / m_tiles;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t r = lane & 15, kg = lane >> 4;
+    const uint32_t col0 = nt * 256 + wave * 32, nch = w.k / 32, nstep = (nch + 3) / 4;
+    const uint32_t lbase = (uint32_t)(uintptr_t)lds;
+    const H16Img& H = a.H;
+    const uint32_t rt0 = mt * 2, rt1 = min(mt * 2 + 1, H.rts - 1);
+
+    // ---- DMA: the activation tile of step q (16 pieces of 1 KiB), its scales and sums ----
+    const uint8_t* const s0 = a.h16 + H.s_off + (size_t)rt0 * nstep * 512;
+    auto issue_b = [&](uint32_t q, uint32_t slot) {
+        const uint32_t qc = min(q, nstep - 1), to = lbase + slot * Y::kBSlot;
+        const uint32_t c = min(qc * 4 + (wave >> 1), nch - 1);
+        dma16(a.h16 + ((size_t)rt0 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to + wave * 1024);
+        dma16(a.h16 + ((size_t)rt1 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to + 8192 + wave * 1024);
+        // scales: chunks 2p, 2p + 1 of a row tile (repeats are the same bytes)
+        const uint32_t i = (wave >> 1) & 1, p = wave & 1, cs = min(qc * 4 + 2 * p + (lane >> 5), nch - 1);
+        dma16(a.h16 + H.d_off + (size_t)(i ? rt1 : rt0) * nch * 512, cs * 512 + (lane & 31) * 16,
+              to + Y::kSc + i * 2048 + p * 1024);
+        if constexpr (T::kMin32)  // 512 bytes of each row tile
+            dma16(s0 + qc * 512,
+                  (lane >> 5 ? (rt1 - rt0) * nstep * 512 : 0u) + (lane & 31) * 16, to + Y::kMs);
+    };
+    WOff<DT> wo;
+    weight_offsets<DT>(wo, w, col0, lane);
+    const uint32_t wls = Y::kOffW + wave * (2 * T::kSlot);
+    auto issue_w = [&](uint32_t st, uint32_t slot) {
+        issue_weights<DT, DV>(wo, w, min(st, nstep - 1), lbase + wls + slot * T::kSlot);
+    };
+    constexpr int kND = (T::kPlaneD && !DV) ? T::kNI : T::kND;
+
+    // lane's operand B in a row tile's (chunk) 2 KiB: row group rg, elements 8 kg ..
+    const uint32_t b_off = (kg & 1) * 1024 + (kg >> 1) * 512 + r * 16;
+    // scales and sums: the row's 8 bytes for kg == 0, a zero entry (half 1) else
+    const uint32_t s_off = kg == 0 ? r * 8 : 256 + r * 8, s_step = kg == 0 ? 128 : 0;
+
+    f4v out[2][4], mid[2][4];  // [column tile][row group]
+
+    // The output tile, stored (first) or added to.  Long K adds to it every 16
+    // steps: a last level of the sum that needs no registers.
+    auto flush = [&](bool first) __attribute__((always_inline)) {
+        uint32_t r0 = r;
+        asm volatile("" : "+v"(r0));  // keeps the addresses out of the step loop's registers
+#pragma unroll
+        for (int rg = 0; rg < 4; rg++) {
+            const uint32_t row = mt * 64 + rg * 16 + r0;
+            if (row >= m) continue;
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) {
+                const uint32_t n = col0 + ct * 16 + 4 * kg;
+                float* yr = y + (size_t)row * w.n + n;
+                const f4v& v = out[ct][rg];
+                if (n + 3 < w.n && (w.n & 3) == 0) {
+                    float4 o = make_float4(v[0], v[1], v[2], v[3]);
+                    if (!first) {
+                        const float4 z = *reinterpret_cast<const float4*>(yr);
+                        o = make_float4(o.x + z.x, o.y + z.y, o.z + z.z, o.w + z.w);
+                    }
+                    *reinterpret_cast<float4*>(yr) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        if (n + e < w.n) yr[e] = first ? v[e] : yr[e] + v[e];
+                }
+            }
+        }
+    };
+
+    issue_b(0, 0);
+    issue_w(0, 0);
+    issue_b(1, 1);
+    issue_w(1, 1);
+    uint32_t slot = 0, free_slot = 2;
+    auto step = [&](uint32_t s) __attribute__((always_inline)) {
+        // step s has landed (step s + 1's DMA is younger), and every wavefront is past step s - 1
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB + kND) : "memory");
+        issue_b(s + 2, free_slot);
+        const uint8_t* bs = lds + slot * Y::kBSlot;
+        const uint8_t* ws = lds + wls + (s & 1) * T::kSlot;
+        uint2 wv[2], b32[4];
+        uint32_t qh[2];
+        h8 A[2][2];  // [chunk & 1][column tile]
+        constexpr int kAhead = T::kMin32 ? 1 : 2, kRingB = kAhead + 1;  // operand reads ahead of their unit
+        uint4 b[kRingB];
+        uint2 bd[kRingB];
+        struct {
+            f4v I[2], sc[2], p[2];
+        } un[2];
+        f4v t[2][4];
+        auto read_b = [&](int u) {
+            const int j = u >> 2, rg = u & 3;
+            b[u % kRingB] = *reinterpret_cast<const uint4*>(bs + (rg >> 1) * 8192 + j * 2048 + (rg & 1) * 256 + b_off);
+            bd[u % kRingB] = *reinterpret_cast<const uint2*>(bs + Y::kSc + (rg >> 1) * 2048 + j * 512 + (rg & 1) * s_step + s_off);
+        };
+        auto read_w = [&](int j) {
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) read_chunk8<DT>(wv[ct], qh[ct], ws, ct * 16 + r, j, kg);
+        };
+        auto grow = [&](int j) {
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) A[j & 1][ct] = expand8<DT>(wv[ct], qh[ct], kg);
+        };
+        read_w(0);
+        read_b(0);
+        // d_w (and m) of the lane's two columns, chunks 0 .. 3: operands of the rank-1
+        // products (only lanes kg == 0 hold them)
+        uint32_t dv[2][4], mv[2][4];
+#pragma unroll
+        for (int ct = 0; ct < 2; ct++) {
+            const uint32_t c = ct * 16 + r;
+            if constexpr (T::kPlaneD && DV) {
+                const uint2 v = *reinterpret_cast<const uint2*>(ws + T::kNI * 1024 + c * 8);
+                const uint32_t x = kg == 0 ? v.x : 0u, z = kg == 0 ? v.y : 0u;
+                dv[ct][0] = x & 0xffffu; dv[ct][1] = x >> 16; dv[ct][2] = z & 0xffffu; dv[ct][3] = z >> 16;
+            } else if constexpr (T::kPlaneD) {
+                const uint16_t* dp = reinterpret_cast<const uint16_t*>(w.d + min(col0 + c, w.n - 1) * w.d_row);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t v = dp[min(s * 4 + j, nch - 1)];
+                    dv[ct][j] = kg == 0 && s * 4 + j < nch ? v : 0u;
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t f = *reinterpret_cast<const uint32_t*>(ws + c * T::kSeg + j * (int)raw_stride(DT));
+                    const uint32_t v = kg == 0 && s * 4 + j < nch ? f : 0u;
+                    dv[ct][j] = v & 0xffffu;
+                    mv[ct][j] = j & 1 ? v & 0xffff0000u : v >> 16;
+                }
+            }
+        }
+        if constexpr (T::kMin32) {
+#pragma unroll
+            for (int rg = 0; rg < 4; rg++)
+                b32[rg] = *reinterpret_cast<const uint2*>(bs + Y::kMs + (rg >> 1) * 512 + (rg & 1) * s_step + s_off);
+        }
+        if (kAhead > 1) read_b(1);
+        grow(0);
+        read_w(1);
+        auto fold = [&](int u) {
+            const int j = u >> 2, rg = u & 3;
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    float x = j == 0 ? 0.f : t[ct][rg][e];
+                    const float I = un[u & 1].I[ct][e], sc = un[u & 1].sc[ct][e];
+                    if constexpr (T::kMin32) {
+                        // per block, as the reference's vec_dot: the min and main terms cancel
+                        const float v = fmaf(I, sc, un[u & 1].p[ct][e]);
+                        x = j == 0 ? v : x + v;
+                    } else {
+                        x = j == 0 ? I * sc : fmaf(I, sc, x);
+                    }
+                    t[ct][rg][e] = x;
+                    if (j == 3) mid[ct][rg][e] += x;
+                }
+        };
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 16; u++) {  // unit u: chunk u / 4, row group u % 4
+            const int j = u >> 2, rg = u & 3;
+            if (u + kAhead < 16) read_b(u + kAhead);
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) {
+                un[u & 1].I[ct] = mfma16x16x32(A[j & 1][ct], as_h8(b[u % kRingB]));
+                un[u & 1].sc[ct] = mfma16x16x16(make_uint2(dv[ct][j], 0), bd[u % kRingB]);
+                if constexpr (T::kMin32)
+                    un[u & 1].p[ct] = mfma16x16x16(j < 2 ? make_uint2(mv[ct][j], 0) : make_uint2(0, mv[ct][j]), b32[rg]);
+            }
+            if (rg == 2 && j < 3) grow(j + 1);
+            if (rg == 3 && j < 2) read_w(j + 2);
+            if (u > 0) fold(u - 1);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        fold(15);
+        // this step's weights are read; fetch step s + 2 over them
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        issue_w(s + 2, s & 1);
+        free_slot = slot;
+        slot = slot == 2 ? 0 : slot + 1;
+    };
+    for (uint32_t s16 = 0; s16 < nstep; s16 += 16) {
+        const uint32_t e16 = min(s16 + 16, nstep);
+#pragma unroll
+        for (int i = 0; i < 8; i++) out[i >> 2][i & 3] = f4v{};
+        for (uint32_t s4 = s16; s4 < e16; s4 += 4) {
+            const uint32_t e4 = min(s4 + 4, e16);
+#pragma unroll
+            for (int i = 0; i < 8; i++) mid[i >> 2][i & 3] = f4v{};
+            for (uint32_t s = s4; s < e4; s++) step(s);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) out[i >> 2][i & 3][e] += mid[i >> 2][i & 3][e];
+        }
+        flush(s16 == 0);
+    }
+    wait_vm<0>();  // no DMA outlives the workgroup's LDS
+}
+
+template <int DT, int TM, bool DV>
+hipError_t launch_ksplit(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    using T = HT<DT>;
+    constexpr int kWaveLds = 3 * T::kSlot + T::kDl, kRed = kWaves * TM * 4 * 64 * 16;
+    constexpr int kLds = kWaves * kWaveLds > kRed ? kWaves * kWaveLds : kRed;
+    const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_ksplit_kernel<DT, TM, DV>), kLds);
+    if (e != hipSuccess) return e;
+    const uint32_t n_tiles = (w.n + 31) / 32, rts = (uint32_t)((m + 31) / 32), m_tiles = (rts + TM - 1) / TM;
+    const uint32_t grid = (m_tiles * n_tiles + 7) / 8 * 8;
+    h16_ksplit_kernel<DT, TM, DV><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+    return hipGetLastError();
+}
+
+template <int DT, bool DV>
+hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    // K split over the wavefronts of a workgroup (32-row tiles up to one
+    // workgroup per CU, then 64-row tiles) against the 256 x 64 tile, us, graph
+    // steps, K = 4096, Q8_0: N = 1024 m = 256 17.1 / 21.3 / 76, 512 30.5 / 24.6 / 79;
+    // N = 4096 m = 64 15.2 / 19.1 / 73, 128 24.8 / 20.9 / 74, 512 88 / 65 / 77;
+    // N = 14336 m = 128 77 / 67 / 81, 256 146 / 111 / 85.  Q5K: 6144 m = 64 22.7 / 18.1 /
+    // 47, 256 57 / 43 / 50, 512 120 / 83 / 55.  A round of tiles (one per CU) costs the
+    // same however few it holds, a round of 64-row K-split workgroups an eighth
+    // of the products and about 16 us (Q5K 13): the tile pays from 148 (112)
+    // tiles in every round.
+    const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
+    if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
+    const size_t tiles = ((m + 63) / 64) * ((w.n + 255) / 256), rounds = (tiles + 255) / 256;
+    if (tiles < rounds * (HT<DT>::kK ? 112 : 148)) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
+    constexpr int kLds = TLay<DT>::kLds;
+    const uint32_t m_tiles = (uint32_t)((m + 63) / 64), n_tiles = (w.n + 255) / 256, grid = (m_tiles * n_tiles + 7) / 8 * 8;
+    if constexpr (HT<DT>::kK) {
+        const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_super_tile_kernel<DT>), kLds);
+        if (e != hipSuccess) return e;
+        h16_super_tile_kernel<DT><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+    } else {
+        const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_block_tile_kernel<DT, DV>), kLds);
+        if (e != hipSuccess) return e;
+        h16_block_tile_kernel<DT, DV><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool h16_supported(uint32_t dtype) {
+    return dtype == XNQ_Q8_0 || dtype == XNQ_Q4_0 || is_raw_layout(dtype);
+}
+
+hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    if (m == 0 || w.n == 0) return hipSuccess;
+    if (!a.h16 || (size_t)a.H.rts * 32 < m || a.k != w.k) return hipErrorInvalidValue;
+    switch (w.dtype) {
+    case XNQ_Q8_0: return w.nb % 4 == 0 ? launch_h16_dt<XNQ_Q8_0, true>(w, a, m, y, s) : launch_h16_dt<XNQ_Q8_0, false>(w, a, m, y, s);
+    case XNQ_Q4_0: return w.nb % 4 == 0 ? launch_h16_dt<XNQ_Q4_0, true>(w, a, m, y, s) : launch_h16_dt<XNQ_Q4_0, false>(w, a, m, y, s);
+    case XNQ_Q4_1: return launch_h16_dt<XNQ_Q4_1, true>(w, a, m, y, s);
+    case XNQ_Q5_0: return launch_h16_dt<XNQ_Q5_0, true>(w, a, m, y, s);
+    case XNQ_Q5_1: return launch_h16_dt<XNQ_Q5_1, true>(w, a, m, y, s);
+    case XNQ_Q2K: return launch_h16_dt<XNQ_Q2K, true>(w, a, m, y, s);
+    case XNQ_Q3K: return launch_h16_dt<XNQ_Q3K, true>(w, a, m, y, s);
+    case XNQ_Q5K: return launch_h16_dt<XNQ_Q5K, true>(w, a, m, y, s);
+    }
+    return hipErrorNotSupported;
+}
+
+}  // namespace xnq

@@ -271,6 +271,19 @@ static bool tiled_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
            (forced == 2 || m > skinny_max_rows() || q4k_prefill_early(weight_dtype, m, k));
 }
 
+// Whether m rows take the f16 matrix-core kernels (the activation quantizer
+// then also writes the f16 copy of the rows); like tiled_act a function of the
+// type, m and K only.  K is bounded as for the matvec kernels, whose LDS holds
+// a row image.  The matvec kernels take up to 8 rows in one launch and read
+// the weights again for every further 8; the f16 kernels cost the same from 1
+// to 32 rows.  m = 8 and 16, K = 4096, us, matvec / f16: Q8_0 N = 1024 8.0 / 12.7
+// and 13.2 / 12.7, 14336 22.3 / 28.0 and 41.7 / 28.5; Q4_0 14336 22.8 / 23.5 and
+// 42.7 / 23.5; Q5K 6144 14.1 / 13.7 and 24.5 / 13.8.
+static bool h16_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
+    return forced == 0 && m > 8 && h16_supported(weight_dtype) &&
+           act_img((uint32_t)k, is_kquant(weight_dtype)).row_bytes <= 160 * 1024;
+}
+
 ALayout act_layout(uint32_t weight_dtype, size_t m, size_t k, int forced) {
     ALayout L;
     L.act_dtype = vec_dot_type(weight_dtype);
@@ -283,6 +296,12 @@ ALayout act_layout(uint32_t weight_dtype, size_t m, size_t k, int forced) {
         L.tile_off = L.bytes;
         L.tile = tile_img(m, (uint32_t)k);
         L.bytes = align_up(L.tile_off + L.tile.bytes);
+    }
+    if (h16_act(weight_dtype, m, k, forced)) {
+        L.h16 = true;
+        L.h16_off = L.bytes;
+        L.himg = h16_img(m, (uint32_t)k, L.act_dtype == XNQ_Q8K, L.act_dtype == XNQ_Q8_1);
+        L.bytes = align_up(L.h16_off + L.himg.bytes);
     }
     return L;
 }
@@ -457,12 +476,13 @@ static xnq_status check_mkn(const xnq_qtensor* qt, size_t m, size_t k, size_t n)
 //            group joins at most 16384 columns (the wavefront-split kernel)
 //   m <= 64  skinny int8-MFMA kernel for Q4K / Q6K
 //   larger m tiled int8-MFMA prefill kernel
-// Q8_0 / Q4_0 and the other dtypes always take the matvec kernels.
+// Q8_0 / Q4_0 and the other dtypes: matvec kernels up to 8 rows, f16 MFMA
+// kernels above.
 // XNQ_SKINNY_MIN_ROWS and XNQ_SKINNY_MAX_ROWS override the skinny range for
 // tuning (read once per process); `forced` is xnq_set_route's override as
 // read at the entry point; `group_n` is the joined width of a group (0 for a
 // single weight).
-enum Route { kMatvec, kSkinny, kMfma };
+enum Route { kMatvec, kSkinny, kMfma, kH16 };
 
 static Route pick_route(uint32_t dtype, size_t m, size_t n, size_t k, int forced, size_t group_n = 0) {
     static const size_t skinny_min = env_size("XNQ_SKINNY_MIN_ROWS", 0);
@@ -470,6 +490,7 @@ static Route pick_route(uint32_t dtype, size_t m, size_t n, size_t k, int forced
     if (forced == 1) return kMatvec;
     if (forced == 2) return kMfma;
     if (forced == 3) return kSkinny;
+    if (h16_act(dtype, m, k, forced)) return kH16;
     // measured crossovers (graph steps, µs, matvec against skinny): the
     // matvec kernels' cost jumps from 4 to 5 rows (the 8-row template) and
     // past 8 rows takes a second launch; the skinny kernel's hardly grows
@@ -542,6 +563,8 @@ static xnq_status matmul_preq_impl(const xnq_qtensor* qt, size_t m, size_t k, si
         float* partial = splits > 1 ? reinterpret_cast<float*>((uint8_t*)workspace_dev + off) : nullptr;
         e = r == kMfma ? launch_mfma(w, a, m, splits, dst_dev, partial, (hipStream_t)stream)
                        : launch_skinny(w, a, m, splits, dst_dev, partial, (hipStream_t)stream);
+    } else if (r == kH16) {
+        e = launch_h16(w, a, m, dst_dev, (hipStream_t)stream);
     } else {
         e = launch_matvec(w, a, m, dst_dev, (hipStream_t)stream);
     }
@@ -696,7 +719,12 @@ xnq_status xnq_qtensor_matmul_t_noalloc(const xnq_qtensor* qt, size_t m, size_t 
     if (st) return st;
     const int forced = g_route.load();
     const size_t need = matmul_t_workspace_size_impl(qt, m, forced);
-    if (need > XNQ_NOALLOC_SCRATCH_BYTES)
+    // The f16 route's copy of the rows fills the scratch from fewer rows on than
+    // the row images alone: up to the rows whose images fit, it runs in slabs
+    // (the rows are independent).
+    const bool slabs = need > XNQ_NOALLOC_SCRATCH_BYTES && pick_route(qt->L.dtype, m, n, k, forced) == kH16 &&
+                       act_layout(qt->L.dtype, m, k, 1).bytes <= XNQ_NOALLOC_SCRATCH_BYTES;
+    if (need > XNQ_NOALLOC_SCRATCH_BYTES && !slabs)
         return fail(XNQ_ERR_INVALID,
                     "matmul_t_noalloc: m = %zu needs %zu bytes of scratch, more than the library's static %zu; "
                     "split the rows or use matmul_t_ws",
@@ -709,7 +737,13 @@ xnq_status xnq_qtensor_matmul_t_noalloc(const xnq_qtensor* qt, size_t m, size_t 
     if (st) return st;
     // every kernel writes the scratch it reads (activation image, split-K
     // partials) before reading it, so nothing needs clearing between calls
-    return matmul_t_ws_impl(qt, m, k, n, lhs_dev, ws, XNQ_NOALLOC_SCRATCH_BYTES, dst_dev, stream, forced);
+    if (!slabs) return matmul_t_ws_impl(qt, m, k, n, lhs_dev, ws, XNQ_NOALLOC_SCRATCH_BYTES, dst_dev, stream, forced);
+    size_t rows = 32;
+    while (matmul_t_workspace_size_impl(qt, 2 * rows, forced) <= XNQ_NOALLOC_SCRATCH_BYTES) rows *= 2;
+    for (size_t i = 0; i < m && !st; i += rows)
+        st = matmul_t_ws_impl(qt, m - i < rows ? m - i : rows, k, n, lhs_dev + i * k, ws, XNQ_NOALLOC_SCRATCH_BYTES,
+                              dst_dev + i * n, stream, forced);
+    return st;
 }
 
 // ---------------------------------------------------------------------------
@@ -897,7 +931,7 @@ static bool mlp_fused(const xnq_qtensor* gate, const xnq_qtensor* up, const xnq_
     if (gate->L.n != up->L.n || !skinny_group(pair, 2, m, forced)) return false;
     if (down->device != gate->device || !is_kquant(down->L.dtype) || fused_route(down, m, forced)) return false;
     const ALayout L = act_layout(down->L.dtype, m, down->L.k, forced);
-    return L.act_dtype == XNQ_Q8K && !L.tiled && down->L.k % 256 == 0;
+    return L.act_dtype == XNQ_Q8K && !L.tiled && !L.h16 && down->L.k % 256 == 0;
 }
 
 static size_t mlp_ws_impl(const xnq_qtensor* gate, const xnq_qtensor* up, const xnq_qtensor* down, size_t m,

@@ -147,6 +147,33 @@ __host__ __device__ inline TileImg tile_img(size_t m, uint32_t k) {
     return T;
 }
 
+// f16 copy of the quantized rows for the f16 matrix-core kernels (k_h16.hip),
+// in MFMA operand order: rows in tiles of 32 (the last one padded with zero
+// rows), lane = 32 * half + row, every piece one contiguous KiB (or less):
+//   quants  [tile][chunk c][step 2][lane 64][16]: elements 16 half + 8 step ..
+//           + 7 of the chunk as f16 whole numbers
+//   32-element activations (Q8_0 / Q8_1 blocks), nst = ceil(nch / 4):
+//     d     [tile][chunk][lane 64][8]: {f16 scale, 0, 0, 0} for half 0, zeros for half 1
+//     s     [tile][4-chunk stage][lane 64][8] (Q4_1, Q5_1 only): Q8_1's f16 s of the
+//           stage's four chunks for half 0, 0 for half 1
+//   Q8K activations:
+//     d     [tile][super-block][row 32] f32
+//     s     [tile][super-block][lane 64][16]: bsums 8 half .. 8 half + 7 as f16
+struct H16Img {
+    uint32_t rts = 0;  // 32-row tiles
+    size_t d_off = 0, s_off = 0, bytes = 0;
+};
+
+__host__ __device__ inline H16Img h16_img(size_t m, uint32_t k, bool kquant, bool mins32) {
+    H16Img H;
+    H.rts = (uint32_t)((m + 31) / 32);
+    const size_t nch = k / 32, nst = (nch + 3) / 4;
+    H.d_off = H.rts * nch * 2048;
+    H.s_off = H.d_off + (kquant ? H.rts * (nch / 8) * 128 : H.rts * nch * 512);
+    H.bytes = H.s_off + (kquant ? H.rts * (nch / 8) * 1024 : mins32 ? H.rts * nst * 512 : 0);
+    return H;
+}
+
 struct ALayout {
     uint32_t act_dtype = 0;
     size_t m = 0, k = 0, bytes = 0;
@@ -154,6 +181,9 @@ struct ALayout {
     bool tiled = false;  // a TileImg follows the row images at tile_off
     size_t tile_off = 0;
     TileImg tile{};
+    bool h16 = false;  // an H16Img follows the row images at h16_off
+    size_t h16_off = 0;
+    H16Img himg{};
 };
 
 struct AView {
@@ -162,6 +192,8 @@ struct AView {
     ActImg A;
     const uint8_t* tile;  // null unless the layout is tiled
     TileImg T;
+    const uint8_t* h16;  // null unless the layout has the f16 copy
+    H16Img H;
 };
 
 // Weights that share one activation row in a decode launch (matvec
@@ -211,6 +243,8 @@ inline AView make_aview(const ALayout& L, const void* base) {
     v.A = L.img;
     v.tile = L.tiled ? v.img + L.tile_off : nullptr;
     v.T = L.tile;
+    v.h16 = L.h16 ? v.img + L.h16_off : nullptr;
+    v.H = L.himg;
     return v;
 }
 
@@ -282,5 +316,9 @@ bool prefill_supported(uint32_t dtype, size_t m, size_t n, size_t k);
 uint32_t prefill_splits(size_t m, size_t n, size_t k);
 hipError_t launch_prefill(const WView& w, const AView& a, size_t m, uint32_t splits, float* y, float* partial,
                           hipStream_t s);
+
+// k_h16.hip: the f16 matrix-core kernels of the other weight types
+bool h16_supported(uint32_t dtype);
+hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s);
 
 }  // namespace xnq
