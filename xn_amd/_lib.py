@@ -78,6 +78,8 @@ class XnqError(RuntimeError):
 def load(path: str | None = None) -> ctypes.CDLL:
     """Load libxnq.so (built in-tree by __graft_entry__.build()) and declare its ABI."""
     global _lib
+    if _lib is not None and path is None:
+        return _lib
     with _lock:
         if _lib is not None and path is None:
             return _lib

@@ -90,7 +90,14 @@ def vec_dot_type(dtype: GgmlDType) -> GgmlDType:
     return GgmlDType.Q8K
 
 
+# The current stream's handle by device index, without the Stream object that
+# torch.cuda.current_stream builds (0.07 against 1.9 us a call).
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device: torch.device) -> int:
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 
@@ -188,8 +195,9 @@ class QTensor:
             raise XnqError(1, f"{dtype.name} tensor {shape}: expected {expect} bytes, got {buf.nbytes}")
         out = ctypes.c_void_p()
         dev = torch.device("cuda", idx)
-        check(_lib.load().xnq_qtensor_upload(idx, int(dtype), buf.ctypes.data, n, k, _stream(dev),
-                                             ctypes.byref(out)))
+        # (the first use of the device in a process may be this one)
+        stream = torch.cuda.current_stream(dev).cuda_stream
+        check(_lib.load().xnq_qtensor_upload(idx, int(dtype), buf.ctypes.data, n, k, stream, ctypes.byref(out)))
         return cls(QStorage(out.value, dev), shape)
 
     @classmethod
@@ -255,9 +263,11 @@ class QTensor:
             raise XnqError(1, f"unexpected lhs length {lhs.numel()} {(m, k, n)}")
         if dst.numel() < m * n:
             raise XnqError(1, f"dst too small ({dst.numel()} < {m * n})")
-        for t, name in ((lhs, "lhs"), (dst, "dst")):
-            if t.device != self.device or t.dtype != torch.float32 or not t.is_contiguous():
-                raise XnqError(1, f"{name} must be a contiguous float32 tensor on {self.device}")
+        dev = self.storage.device
+        if lhs.device != dev or lhs.dtype is not torch.float32 or not lhs.is_contiguous():
+            raise XnqError(1, f"lhs must be a contiguous float32 tensor on {dev}")
+        if dst.device != dev or dst.dtype is not torch.float32 or not dst.is_contiguous():
+            raise XnqError(1, f"dst must be a contiguous float32 tensor on {dev}")
         return m, k, n
 
     def matmul_t(self, mkn: Tuple[int, int, int], lhs: torch.Tensor, dst: torch.Tensor) -> None:
@@ -269,14 +279,18 @@ class QTensor:
         device allocation) and the library runs quantize_lhs + T::matmul, as
         k_quants::matmul does.  Runs on the current stream."""
         m, k, n = self._check_mm(mkn, lhs, dst)
+        self._matmul_t(m, k, n, lhs, dst)
+
+    def _matmul_t(self, m: int, k: int, n: int, lhs: torch.Tensor, dst: torch.Tensor) -> None:
+        """matmul_t on checked operands."""
         if m == 0 or n == 0:
             return
         L = _lib.load()
-        h = self.storage.handle
+        h, dev = self.storage._h, self.storage.device
         nbytes = L.xnq_qtensor_matmul_t_workspace_size(h, m)
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=self.device) if nbytes else None
-        check(L.xnq_qtensor_matmul_t_ws(h, m, k, n, _ptr(lhs), _ptr(ws) if ws is not None else None, nbytes,
-                                        _ptr(dst), _stream(self.device)))
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+        check(L.xnq_qtensor_matmul_t_ws(h, m, k, n, lhs.data_ptr(), ws.data_ptr() if nbytes else None, nbytes,
+                                        dst.data_ptr(), _stream(dev)))
 
     def matmul_t_workspace_size(self, m: int) -> int:
         """Bytes of caller scratch matmul_t_ws needs for m rows (0 on the fused decode route)."""
@@ -345,19 +359,23 @@ class QLinear:
 
     def forward(self, xs: torch.Tensor) -> torch.Tensor:
         """mod.rs:352-384: (..., k) -> (..., n), then + bias."""
-        dims = self.weight.shape()
+        weight = self.weight
+        dims, shape = weight._shape, xs.shape
         if len(dims) != 2:
             raise XnqError(1, f"unexpected rank, expected: 2, got: {len(dims)} ({dims})")
         n, k = dims
-        if xs.dim() < 2:
-            raise XnqError(1, f"input tensor has only one dimension {tuple(xs.shape)}")
-        if xs.shape[-1] != k:
-            raise XnqError(1, f"input tensor {tuple(xs.shape)} incompatible with {list(dims)}")
-        dst_shape = tuple(xs.shape[:-1]) + (n,)
-        dst = torch.empty(dst_shape, dtype=torch.float32, device=self.weight.device)
+        if len(shape) < 2:
+            raise XnqError(1, f"input tensor has only one dimension {tuple(shape)}")
+        if shape[-1] != k:
+            raise XnqError(1, f"input tensor {tuple(shape)} incompatible with {list(dims)}")
+        dev = weight.storage.device
+        dst = torch.empty(shape[:-1] + (n,), dtype=torch.float32, device=dev)
         xs = xs.contiguous()
         m = xs.numel() // k
-        self.weight.matmul_t((m, k, n), xs, dst)
+        if xs.dtype is torch.float32 and xs.device == dev:
+            weight._matmul_t(m, k, n, xs, dst)  # nothing of matmul_t's checks can fail
+        else:
+            weight.matmul_t((m, k, n), xs, dst)
         if self.bias is not None:
             dst = dst + self.bias
         return dst
@@ -446,12 +464,13 @@ def matmul_t_group(qts, m: int, k: int, lhs: torch.Tensor, dsts) -> None:
     for qt, d in zip(qts, dsts):
         qt._check_mm((m, k, qt.shape()[0]), lhs, d)
     L = _lib.load()
-    hs = (ctypes.c_void_p * max(len(qts), 1))(*[qt.storage.handle for qt in qts])
+    dev = lhs.device
+    hs = (ctypes.c_void_p * max(len(qts), 1))(*[qt.storage._h.value for qt in qts])
     ds = (ctypes.c_void_p * max(len(dsts), 1))(*[d.data_ptr() for d in dsts])
     nbytes = L.xnq_matmul_t_group_workspace_size(hs, len(qts), m)
-    ws = torch.empty(nbytes, dtype=torch.uint8, device=lhs.device) if nbytes else None
-    check(L.xnq_matmul_t_group(hs, len(qts), m, k, _ptr(lhs), ds, _ptr(ws) if ws is not None else None, nbytes,
-                               _stream(lhs.device)))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=dev) if nbytes else None
+    check(L.xnq_matmul_t_group(hs, len(qts), m, k, lhs.data_ptr(), ds, ws.data_ptr() if nbytes else None, nbytes,
+                               _stream(dev)))
 
 
 # -- stream capture (cuda_backend/mod.rs:251-283: capture_begin / capture_end) --
