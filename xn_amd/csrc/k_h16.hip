@@ -550,31 +550,29 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
 }
 
 // ---------------------------------------------------------------------------
-// Prefill sizes: a workgroup of eight wavefronts owns 256 weight columns and
-// 64 rows; wavefront w owns columns 32w .. 32w+31 and every row, so each
-// weight is expanded once per workgroup, and the activation tile is shared
-// through LDS.  K advances four chunks (128) a step.  All data moves by LDS
-// DMA: the activation tile (1 KiB pieces, shared) into a three-slot ring two
-// steps ahead, each wavefront's own weights into two slots one stage ahead.
-// One barrier per step publishes the shared pieces; each wavefront waits for
-// its own DMA by exact count.
+// Prefill sizes: a workgroup owns 256 weight columns and 64 rows, K advances
+// four chunks (128) a step, and the activation tile is shared through LDS.  All
+// data moves by LDS DMA; one barrier per step publishes the shared pieces, and
+// each wavefront waits for its own DMA by exact count.
 //
-// K types (this kernel): 32 x 32 tiles, a stage is a super-block and two steps.
+// The K types: eight wavefronts; wavefront w owns columns 32w .. 32w+31 and
+// every row, so each weight is expanded once per workgroup.  The activation
+// tile (1 KiB pieces) goes into a three-slot ring two steps ahead, each
+// wavefront's own weights (a super-block, two steps) into two slots one
+// super-block ahead.
 // ---------------------------------------------------------------------------
 template <int DT>
 struct TLay {
     using T = HT<DT>;
-    static constexpr int kBSlot = 2 * 4 * 2048 + (T::kK ? 0 : 2 * 2048 + (T::kMin32 ? 2 * 512 : 0));  // quants (, scales, sums)
-    static constexpr int kSc = 2 * 4 * 2048, kMs = kSc + 2 * 2048;  // offsets in a slot
-    static constexpr int kSb = T::kK ? 2 * 128 + (T::kMinK ? 2 * 1024 : 0) : 0;  // a super-block's d_a, sums
+    static constexpr int kBSlot = 2 * 4 * 2048;
+    static constexpr int kSb = 2 * 128 + (T::kMinK ? 2 * 1024 : 0);  // a super-block's d_a, sums
     static constexpr int kOffW = 3 * kBSlot;
     static constexpr int kOffSb = kOffW + kWaves * 2 * T::kSlot;
     static constexpr int kOffDl = kOffSb + 2 * kSb;
     static constexpr int kLds = kOffDl + kWaves * T::kDl;
     static_assert(kLds <= 160 * 1024, "LDS budget");
     // DMA instructions of every wavefront: per step, and per super-block
-    static constexpr int kNB = 2 + (T::kK ? 0 : 1) + (T::kMin32 ? 1 : 0);
-    static constexpr int kNSb = T::kK ? 1 + (T::kMinK ? 1 : 0) : 0;
+    static constexpr int kNB = 2, kNSb = 1 + (T::kMinK ? 1 : 0);
 };
 
 template <int DT>
@@ -699,64 +697,47 @@ __global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView
 }
 
 // ---------------------------------------------------------------------------
-// The 32-element types at prefill sizes, on 16 x 16 tiles: one K = 32 product
-// is one chunk, and the four sums and four scales of a tile take 8 registers,
-// so the products of one row group are in flight while the previous one's are
-// folded, within the 256 registers that two wavefronts per SIMD leave each.
-// (On 32 x 32 tiles the same pipeline needs 96 registers and spills, and a
-// spill's reload waits for every DMA in flight.)
+// The 32-element types at prefill sizes.  A unit (32 x 32 x 32) is 3 MFMAs, 20
+// vector operations to fold it, and 20 to 24 (Q5: 40) to expand its weights: the
+// vector units bound it (1.8 ns an operation beside MFMAs, 14 ns an MFMA), and
+// two wavefronts per SIMD left them idle while both waited (LDS 33 % of the
+// time).  So sixteen wavefronts, four per SIMD, with one 32 x 32 tile each (a
+// column group's weights are fetched once for its two wavefronts and expanded
+// by both): M = 512, 4096 -> 14336, one box, us a step with the quantizer, 8
+// wavefronts of 32 x 64 on 16 x 16 tiles / this: Q4_0 162 / 148, Q8_0 161 / 145.
+// Three slots of LDS where they fit, fetched two steps ahead, else two.
 // ---------------------------------------------------------------------------
-typedef float f4v __attribute__((ext_vector_type(4)));
-
 template <int DT>
-__device__ __forceinline__ void read_chunk8(uint2& v, uint32_t& qh, const uint8_t* slot, uint32_t c, int j, uint32_t kg) {
-    const uint8_t* col = slot + c * HT<DT>::kSeg;
-    const uint32_t o = 8 * (kg & 1);
-    if constexpr (DT == XNQ_Q8_0) {
-        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, 2 * j + (kg >> 1)) + o);
-    } else if constexpr (DT == XNQ_Q4_0) {
-        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, j) + o);
-    } else if constexpr (DT == XNQ_Q4_1) {
-        const uint32_t* p = reinterpret_cast<const uint32_t*>(col + j * 20 + 4 + o);
-        v = make_uint2(p[0], p[1]);
-    } else {
-        v = *reinterpret_cast<const uint2*>(col + j * 24 + 8 + o);
-        qh = *reinterpret_cast<const uint32_t*>(col + j * 24 + 4);
-    }
-}
+struct BLay {
+    using T = HT<DT>;
+    static constexpr int kSc = 2 * 4 * 2048, kMs = kSc + 2 * 2048;  // scales, sums: offsets in a slot
+    static constexpr int kBSlot = kMs + (T::kMin32 ? 2 * 512 : 0);
+    static constexpr int kWSlot = 8 * T::kSlot;
+    static constexpr int kSlots = 3 * (kBSlot + kWSlot) <= 160 * 1024 ? 3 : 2;
+    static constexpr int kOffW = kSlots * kBSlot, kLds = kOffW + kSlots * kWSlot;
+    static_assert(kLds <= 160 * 1024, "LDS budget");
+};
 
-template <int DT>
-__device__ __forceinline__ h8 expand8(const uint2& v, uint32_t qh, uint32_t kg) {
-    const uint32_t d[2] = {v.x, v.y};
-    h2 q[4];
-    const h2 b = splat2(DT == XNQ_Q8_0 ? -1152.f : DT == XNQ_Q4_0 ? -1032.f : DT == XNQ_Q5_0 ? -1040.f : -1024.f);
-#pragma unroll
-    for (int i = 0; i < 2; i++) {
-        uint32_t x;
-        if constexpr (DT == XNQ_Q8_0) {
-            x = d[i] ^ 0x80808080u;
-        } else {
-            x = (d[i] >> (4 * (kg >> 1))) & 0x0F0F0F0Fu;
-            if (DT == XNQ_Q5_0 || DT == XNQ_Q5_1) x |= spread_bit4((qh >> (8 * kg + 4 * i)) & 15u);
-        }
-        q[2 * i] = magic01(x) + b;
-        q[2 * i + 1] = magic23(x) + b;
+// s_waitcnt vmcnt(n) for a wavefront-uniform n of 1 .. 8
+__device__ __forceinline__ void wait_vm_n(uint32_t n) {
+    switch (n) {
+    case 1: wait_vm<1>(); break;
+    case 2: wait_vm<2>(); break;
+    case 3: wait_vm<3>(); break;
+    case 4: wait_vm<4>(); break;
+    case 5: wait_vm<5>(); break;
+    case 6: wait_vm<6>(); break;
+    case 7: wait_vm<7>(); break;
+    case 8: wait_vm<8>(); break;
+    default: wait_vm<0>(); break;
     }
-    return h8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
-}
-
-__device__ __forceinline__ f4v mfma16x16x32(h8 a, h8 b) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f4v{}, 0, 0, 0);
-}
-__device__ __forceinline__ f4v mfma16x16x16(uint2 a, uint2 b) {
-    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), f4v{}, 0, 0, 0);
 }
 
 template <int DT, bool DV>
-__global__ __launch_bounds__(kThreads) void h16_block_tile_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
-                                                                  uint32_t n_tiles, float* __restrict__ y) {
+__global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
+                                                              uint32_t n_tiles, float* __restrict__ y) {
     using T = HT<DT>;
-    using Y = TLay<DT>;
+    using Y = BLay<DT>;
     extern __shared__ __align__(16) uint8_t lds[];
     const uint32_t total = m_tiles * n_tiles, per = (total + 7) / 8;
     const uint32_t wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // one XCD: consecutive items, which share columns
@@ -764,199 +745,134 @@ __global__ __launch_bounds__(kThreads) void h16_block_tile_kernel(WView w, AView
     const uint32_t mt = wi % m_tiles, nt = wi / m_tiles;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t r = lane & 15, kg = lane >> 4;
-    const uint32_t col0 = nt * 256 + wave * 32, nch = w.k / 32, nstep = (nch + 3) / 4;
+    const uint32_t cw = wave & 7, rh = wave >> 3;  // column group, row tile
+    const uint32_t lrow = lane & 31, g = lane >> 5;
+    const uint32_t col0 = nt * 256 + cw * 32, nch = w.k / 32, nstep = (nch + 3) / 4;
     const uint32_t lbase = (uint32_t)(uintptr_t)lds;
     const H16Img& H = a.H;
     const uint32_t rt0 = mt * 2, rt1 = min(mt * 2 + 1, H.rts - 1);
 
-    // ---- DMA: the activation tile of step q (16 pieces of 1 KiB), its scales and sums ----
-    const uint8_t* const s0 = a.h16 + H.s_off + (size_t)rt0 * nstep * 512;
-    auto issue_b = [&](uint32_t q, uint32_t slot) {
-        const uint32_t qc = min(q, nstep - 1), to = lbase + slot * Y::kBSlot;
-        const uint32_t c = min(qc * 4 + (wave >> 1), nch - 1);
-        dma16(a.h16 + ((size_t)rt0 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to + wave * 1024);
-        dma16(a.h16 + ((size_t)rt1 * nch + c) * 2048 + (wave & 1) * 1024, lane * 16, to + 8192 + wave * 1024);
-        // scales: chunks 2p, 2p + 1 of a row tile (repeats are the same bytes)
-        const uint32_t i = (wave >> 1) & 1, p = wave & 1, cs = min(qc * 4 + 2 * p + (lane >> 5), nch - 1);
-        dma16(a.h16 + H.d_off + (size_t)(i ? rt1 : rt0) * nch * 512, cs * 512 + (lane & 31) * 16,
-              to + Y::kSc + i * 2048 + p * 1024);
-        if constexpr (T::kMin32)  // 512 bytes of each row tile
-            dma16(s0 + qc * 512,
-                  (lane >> 5 ? (rt1 - rt0) * nstep * 512 : 0u) + (lane & 31) * 16, to + Y::kMs);
-    };
     WOff<DT> wo;
     weight_offsets<DT>(wo, w, col0, lane);
-    const uint32_t wls = Y::kOffW + wave * (2 * T::kSlot);
-    auto issue_w = [&](uint32_t st, uint32_t slot) {
-        issue_weights<DT, DV>(wo, w, min(st, nstep - 1), lbase + wls + slot * T::kSlot);
+    // DMA of step q: one 1 KiB piece of the activation tile per wavefront, the
+    // scales from wavefronts 0 .. 3, the sums from 4, a column group's weights
+    // from its two wavefronts in turn
+    const uint8_t* const b0 = a.h16 + (size_t)(rh ? rt1 : rt0) * nch * 2048 + (cw & 1) * 1024;
+    const uint8_t* const d0 = a.h16 + H.d_off + (size_t)(wave >> 1 ? rt1 : rt0) * nch * 512;
+    const uint8_t* const s0 = a.h16 + H.s_off + (size_t)rt0 * nstep * 512;
+    auto issue = [&](uint32_t q, uint32_t slot) {
+        const uint32_t to = lbase + slot * Y::kBSlot, tw = lbase + Y::kOffW + slot * Y::kWSlot + cw * T::kSlot;
+        const uint32_t qc = min(q, nstep - 1);
+        dma16(b0 + (size_t)min(qc * 4 + (cw >> 1), nch - 1) * 2048, lane * 16, to + wave * 1024);
+        if (wave < 4)
+            dma16(d0, min(qc * 4 + 2 * (wave & 1) + g, nch - 1) * 512 + lrow * 16, to + Y::kSc + wave * 1024);
+        if (T::kMin32 && wave == 4) dma16(s0 + qc * 512, (g ? (rt1 - rt0) * nstep * 512 : 0u) + lrow * 16, to + Y::kMs);
+#pragma unroll
+        for (int i = 0; i < T::kNI; i++) {
+            if ((i & 1) != (int)rh) continue;
+            uint32_t off = qc * T::kSeg + wo.in[i];
+            if (!(T::kPlaneD && DV)) off = min(off, w.q_row - T::kPB);
+            if (T::kPB == 16) dma16(w.q, wo.row[i] + off, tw + i * 1024);
+            else dma4(w.q, wo.row[i] + off, tw + i * 256);
+        }
+        if (T::kPlaneD && DV && rh == 1) dma4(w.d, wo.d + qc * 8, tw + T::kNI * 1024);
     };
-    constexpr int kND = (T::kPlaneD && !DV) ? T::kNI : T::kND;
+    // this wavefront's DMA instructions of a step
+    const uint32_t nd = 1 + (wave < 4 ? 1 : 0) + (T::kMin32 && wave == 4 ? 1 : 0) + (rh == 0 ? (T::kNI + 1) / 2 : T::kNI / 2) +
+                        (T::kPlaneD && DV && rh == 1 ? 1 : 0);
 
-    // lane's operand B in a row tile's (chunk) 2 KiB: row group rg, elements 8 kg ..
-    const uint32_t b_off = (kg & 1) * 1024 + (kg >> 1) * 512 + r * 16;
-    // scales and sums: the row's 8 bytes for kg == 0, a zero entry (half 1) else
-    const uint32_t s_off = kg == 0 ? r * 8 : 256 + r * 8, s_step = kg == 0 ? 128 : 0;
-
-    f4v out[2][4], mid[2][4];  // [column tile][row group]
+    f16v out, mid;
 
     // The output tile, stored (first) or added to.  Long K adds to it every 16
     // steps: a last level of the sum that needs no registers.
     auto flush = [&](bool first) __attribute__((always_inline)) {
-        uint32_t r0 = r;
+        uint32_t r0 = lrow;
         asm volatile("" : "+v"(r0));  // keeps the addresses out of the step loop's registers
+        const uint32_t row = mt * 64 + rh * 32 + r0;
+        if (row < m) {
+            float* yr = y + (size_t)row * w.n;
 #pragma unroll
-        for (int rg = 0; rg < 4; rg++) {
-            const uint32_t row = mt * 64 + rg * 16 + r0;
-            if (row >= m) continue;
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++) {
-                const uint32_t n = col0 + ct * 16 + 4 * kg;
-                float* yr = y + (size_t)row * w.n + n;
-                const f4v& v = out[ct][rg];
+            for (int q = 0; q < 4; q++) {
+                const uint32_t n = col0 + 4 * g + 8 * q;
                 if (n + 3 < w.n && (w.n & 3) == 0) {
-                    float4 o = make_float4(v[0], v[1], v[2], v[3]);
+                    float4 o = make_float4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+                    float4* p = reinterpret_cast<float4*>(yr + n);
                     if (!first) {
-                        const float4 z = *reinterpret_cast<const float4*>(yr);
+                        const float4 z = *p;
                         o = make_float4(o.x + z.x, o.y + z.y, o.z + z.z, o.w + z.w);
                     }
-                    *reinterpret_cast<float4*>(yr) = o;
+                    *p = o;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (n + e < w.n) yr[e] = first ? v[e] : yr[e] + v[e];
+                        if (n + e < w.n) yr[n + e] = first ? out[4 * q + e] : yr[n + e] + out[4 * q + e];
                 }
             }
         }
     };
 
-    issue_b(0, 0);
-    issue_w(0, 0);
-    issue_b(1, 1);
-    issue_w(1, 1);
-    uint32_t slot = 0, free_slot = 2;
+    issue(0, 0);
+    if (Y::kSlots == 3) issue(1, 1);
+    uint32_t slot = 0;
     auto step = [&](uint32_t s) __attribute__((always_inline)) {
-        // step s has landed (step s + 1's DMA is younger), and every wavefront is past step s - 1
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB + kND) : "memory");
-        issue_b(s + 2, free_slot);
-        const uint8_t* bs = lds + slot * Y::kBSlot;
-        const uint8_t* ws = lds + wls + (s & 1) * T::kSlot;
-        uint2 wv[2], b32[4];
-        uint32_t qh[2];
-        h8 A[2][2];  // [chunk & 1][column tile]
-        constexpr int kAhead = T::kMin32 ? 1 : 2, kRingB = kAhead + 1;  // operand reads ahead of their unit
-        uint4 b[kRingB];
-        uint2 bd[kRingB];
-        struct {
-            f4v I[2], sc[2], p[2];
-        } un[2];
-        f4v t[2][4];
-        auto read_b = [&](int u) {
-            const int j = u >> 2, rg = u & 3;
-            b[u % kRingB] = *reinterpret_cast<const uint4*>(bs + (rg >> 1) * 8192 + j * 2048 + (rg & 1) * 256 + b_off);
-            bd[u % kRingB] = *reinterpret_cast<const uint2*>(bs + Y::kSc + (rg >> 1) * 2048 + j * 512 + (rg & 1) * s_step + s_off);
+        // step s has landed, and every wavefront is past step s - 1, whose slot is filled next
+        if (Y::kSlots == 3) wait_vm_n(nd);
+        else wait_vm<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (Y::kSlots == 3) issue(s + 2, slot == 0 ? 2 : slot - 1);
+        else issue(s + 1, slot ^ 1);
+        const uint8_t* bs = lds + slot * Y::kBSlot + rh * 8192 + lane * 16;
+        const uint8_t* ds = lds + slot * Y::kBSlot + Y::kSc + rh * 2048 + lane * 8;
+        const uint8_t* ws = lds + Y::kOffW + slot * Y::kWSlot + cw * T::kSlot;
+        Scales<DT> S;
+        read_scales<DT, DV>(S, w, ws, nullptr, col0, lane, s, nch);
+        uint2 ms = make_uint2(0, 0);
+        if constexpr (T::kMin32) ms = *reinterpret_cast<const uint2*>(lds + slot * Y::kBSlot + Y::kMs + rh * 512 + lane * 8);
+        // chunk j's products are issued, then chunk j + 1 is expanded beside them, then
+        // chunk j is folded
+        f16v t;
+        h8 A[2][2];
+        Bytes by;
+        uint4 b[2];
+        uint2 bd;
+        auto read_b = [&](int j) {
+            b[0] = *reinterpret_cast<const uint4*>(bs + j * 2048);
+            b[1] = *reinterpret_cast<const uint4*>(bs + j * 2048 + 1024);
+            bd = *reinterpret_cast<const uint2*>(ds + j * 512);
         };
-        auto read_w = [&](int j) {
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++) read_chunk8<DT>(wv[ct], qh[ct], ws, ct * 16 + r, j, kg);
-        };
-        auto grow = [&](int j) {
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++) A[j & 1][ct] = expand8<DT>(wv[ct], qh[ct], kg);
-        };
-        read_w(0);
+        read_chunk<DT>(by, ws, lrow, 0, g);
         read_b(0);
-        // d_w (and m) of the lane's two columns, chunks 0 .. 3: operands of the rank-1
-        // products (only lanes kg == 0 hold them)
-        uint32_t dv[2][4], mv[2][4];
+        expand<DT>(by, 0, g, S.hd, A[0]);
+        read_chunk<DT>(by, ws, lrow, 1, g);
 #pragma unroll
-        for (int ct = 0; ct < 2; ct++) {
-            const uint32_t c = ct * 16 + r;
-            if constexpr (T::kPlaneD && DV) {
-                const uint2 v = *reinterpret_cast<const uint2*>(ws + T::kNI * 1024 + c * 8);
-                const uint32_t x = kg == 0 ? v.x : 0u, z = kg == 0 ? v.y : 0u;
-                dv[ct][0] = x & 0xffffu; dv[ct][1] = x >> 16; dv[ct][2] = z & 0xffffu; dv[ct][3] = z >> 16;
-            } else if constexpr (T::kPlaneD) {
-                const uint16_t* dp = reinterpret_cast<const uint16_t*>(w.d + min(col0 + c, w.n - 1) * w.d_row);
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint32_t v = dp[min(s * 4 + j, nch - 1)];
-                    dv[ct][j] = kg == 0 && s * 4 + j < nch ? v : 0u;
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const uint32_t f = *reinterpret_cast<const uint32_t*>(ws + c * T::kSeg + j * (int)raw_stride(DT));
-                    const uint32_t v = kg == 0 && s * 4 + j < nch ? f : 0u;
-                    dv[ct][j] = v & 0xffffu;
-                    mv[ct][j] = j & 1 ? v & 0xffff0000u : v >> 16;
-                }
+        for (int j = 0; j < 4; j++) {
+            Unit<DT> un;
+            unit_mma<DT>(un, A[j & 1], S, j, b, bd, ms);
+            __builtin_amdgcn_sched_barrier(0);
+            if (j < 3) {
+                read_b(j + 1);
+                expand<DT>(by, j + 1, g, S.hd, A[(j + 1) & 1]);
+                asm volatile("" : "+v"(A[(j + 1) & 1][0]), "+v"(A[(j + 1) & 1][1]));
+                if (j < 2) read_chunk<DT>(by, ws, lrow, j + 2, g);
             }
-        }
-        if constexpr (T::kMin32) {
-#pragma unroll
-            for (int rg = 0; rg < 4; rg++)
-                b32[rg] = *reinterpret_cast<const uint2*>(bs + Y::kMs + (rg >> 1) * 512 + (rg & 1) * s_step + s_off);
-        }
-        if (kAhead > 1) read_b(1);
-        grow(0);
-        read_w(1);
-        auto fold = [&](int u) {
-            const int j = u >> 2, rg = u & 3;
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    float x = j == 0 ? 0.f : t[ct][rg][e];
-                    const float I = un[u & 1].I[ct][e], sc = un[u & 1].sc[ct][e];
-                    if constexpr (T::kMin32) {
-                        // per block, as the reference's vec_dot: the min and main terms cancel
-                        const float v = fmaf(I, sc, un[u & 1].p[ct][e]);
-                        x = j == 0 ? v : x + v;
-                    } else {
-                        x = j == 0 ? I * sc : fmaf(I, sc, x);
-                    }
-                    t[ct][rg][e] = x;
-                    if (j == 3) mid[ct][rg][e] += x;
-                }
-        };
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int u = 0; u < 16; u++) {  // unit u: chunk u / 4, row group u % 4
-            const int j = u >> 2, rg = u & 3;
-            if (u + kAhead < 16) read_b(u + kAhead);
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++) {
-                un[u & 1].I[ct] = mfma16x16x32(A[j & 1][ct], as_h8(b[u % kRingB]));
-                un[u & 1].sc[ct] = mfma16x16x16(make_uint2(dv[ct][j], 0), bd[u % kRingB]);
-                if constexpr (T::kMin32)
-                    un[u & 1].p[ct] = mfma16x16x16(j < 2 ? make_uint2(mv[ct][j], 0) : make_uint2(0, mv[ct][j]), b32[rg]);
-            }
-            if (rg == 2 && j < 3) grow(j + 1);
-            if (rg == 3 && j < 2) read_w(j + 2);
-            if (u > 0) fold(u - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            unit_add<DT>(un, j == 0, t);
+            asm volatile("" : "+v"(t));  // folded here, not at the step's end (four chunks' sums would not fit)
             __builtin_amdgcn_sched_barrier(0);
         }
-        fold(15);
-        // this step's weights are read; fetch step s + 2 over them
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        issue_w(s + 2, s & 1);
-        free_slot = slot;
-        slot = slot == 2 ? 0 : slot + 1;
+#pragma unroll
+        for (int e = 0; e < 16; e++) mid[e] += t[e];
+        slot = slot + 1 == Y::kSlots ? 0 : slot + 1;
     };
     for (uint32_t s16 = 0; s16 < nstep; s16 += 16) {
         const uint32_t e16 = min(s16 + 16, nstep);
-#pragma unroll
-        for (int i = 0; i < 8; i++) out[i >> 2][i & 3] = f4v{};
+        out = f16v{};
         for (uint32_t s4 = s16; s4 < e16; s4 += 4) {
             const uint32_t e4 = min(s4 + 4, e16);
-#pragma unroll
-            for (int i = 0; i < 8; i++) mid[i >> 2][i & 3] = f4v{};
+            mid = f16v{};
             for (uint32_t s = s4; s < e4; s++) step(s);
 #pragma unroll
-            for (int i = 0; i < 8; i++)
-#pragma unroll
-                for (int e = 0; e < 4; e++) out[i >> 2][i & 3][e] += mid[i >> 2][i & 3][e];
+            for (int e = 0; e < 16; e++) out[e] += mid[e];
         }
         flush(s16 == 0);
     }
@@ -991,16 +907,17 @@ hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hip
     if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
     const size_t tiles = ((m + 63) / 64) * ((w.n + 255) / 256), rounds = (tiles + 255) / 256;
     if (tiles < rounds * (HT<DT>::kK ? 112 : 148)) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
-    constexpr int kLds = TLay<DT>::kLds;
     const uint32_t m_tiles = (uint32_t)((m + 63) / 64), n_tiles = (w.n + 255) / 256, grid = (m_tiles * n_tiles + 7) / 8 * 8;
     if constexpr (HT<DT>::kK) {
+        constexpr int kLds = TLay<DT>::kLds;
         const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_super_tile_kernel<DT>), kLds);
         if (e != hipSuccess) return e;
         h16_super_tile_kernel<DT><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
     } else {
+        constexpr int kLds = BLay<DT>::kLds;
         const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_block_tile_kernel<DT, DV>), kLds);
         if (e != hipSuccess) return e;
-        h16_block_tile_kernel<DT, DV><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+        h16_block_tile_kernel<DT, DV><<<grid, 1024, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
     }
     return hipGetLastError();
 }
