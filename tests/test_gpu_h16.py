@@ -1,5 +1,5 @@
 """The f16 matrix-core kernels (k_h16.hip) against the CPU oracle: every type
-they take, at the edges of their tiles (32 and 64 rows, 32 and 256 columns),
+they take, at the edges of their tiles (16, 32 and 64 rows, 32 and 256 columns),
 of their K stages (128 and 256, with the remainders of K), and of the rule
 that chooses between them; tiny (f16 subnormal) scales; infinities and NaN in
 the activations against the matvec kernels; the slabs of matmul_t_noalloc.
@@ -46,6 +46,13 @@ def check(orc, dev, dt, m, k, n, seed, wscale=0.02, xscale=1.0):
 @pytest.mark.parametrize("m,k,n", [(9, 64, 31), (32, 192, 33), (33, 1088, 65), (17, 4160, 96), (64, 2048, 8200)])
 def test_block_types_ksplit(orc, dev, dt, m, k, n):
     check(orc, dev, dt, m, k, n, 100 + dt + m)
+
+
+# 16-row tiles (K of whole stages): one tile at any N, an odd count of them, ragged rows and columns
+@pytest.mark.parametrize("dt", BLOCK32)
+@pytest.mark.parametrize("m,k,n", [(9, 128, 31), (16, 640, 8200), (17, 1152, 33), (47, 4224, 67), (125, 2048, 100)])
+def test_block_types_16_rows(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 150 + dt + m)
 
 
 @pytest.mark.parametrize("dt", [Q4_0, Q8_0])

@@ -550,6 +550,222 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
 }
 
 // ---------------------------------------------------------------------------
+// The same for 16 rows, the 32-element types: a workgroup owns 32 columns and 16
+// rows (the upper or lower half of a 32-row tile of the image) on 16 x 16
+// tiles, where one K = 32 product is one chunk.  A wavefront's stages are a
+// serial chain (activation loads, expansion, products, fold), and a workgroup
+// has the CU's LDS to itself, so what counts is a stage's length: 16 rows halve
+// its activation bytes and products and take a third off its vector work, and
+// 32-row tiles leave CUs idle where these are still one round.  us, graph steps
+// with the quantize, 32-row tiles / this, K = 4096: Q8_0 N = 1024 m = 125 14.8 /
+// 13.1, N = 4096 m = 16 13.4 / 11.8 and 32 13.9 / 12.3, N = 14336 m = 16 29.1 /
+// 26.3; Q4_0 N = 4096 m = 16 12.8 / 11.4; Q4_1 14.4 / 13.3; Q5_0 13.3 / 13.3 and
+// Q5_1 14.5 / 14.5 (their bit planes' expansion is what counts), N = 14336
+// 30.0 / 26.0.
+// ---------------------------------------------------------------------------
+typedef float f4v __attribute__((ext_vector_type(4)));
+
+template <int DT>
+__device__ __forceinline__ void read_chunk8(uint2& v, uint32_t& qh, const uint8_t* slot, uint32_t c, int j, uint32_t kg) {
+    const uint8_t* col = slot + c * HT<DT>::kSeg;
+    const uint32_t o = 8 * (kg & 1);
+    if constexpr (DT == XNQ_Q8_0) {
+        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, 2 * j + (kg >> 1)) + o);
+    } else if constexpr (DT == XNQ_Q4_0) {
+        v = *reinterpret_cast<const uint2*>(slot + piece_off<DT>(c, j) + o);
+    } else if constexpr (DT == XNQ_Q4_1) {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(col + j * 20 + 4 + o);
+        v = make_uint2(p[0], p[1]);
+    } else {
+        v = *reinterpret_cast<const uint2*>(col + j * 24 + 8 + o);
+        qh = *reinterpret_cast<const uint32_t*>(col + j * 24 + 4);
+    }
+}
+
+// lane (column, kg = lane / 16): elements 8 kg .. 8 kg + 7 of a chunk
+template <int DT>
+__device__ __forceinline__ h8 expand8(const uint2& v, uint32_t qh, uint32_t kg) {
+    const uint32_t d[2] = {v.x, v.y};
+    h2 q[4];
+    const h2 b = splat2(DT == XNQ_Q8_0 ? -1152.f : DT == XNQ_Q4_0 ? -1032.f : DT == XNQ_Q5_0 ? -1040.f : -1024.f);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        uint32_t x;
+        if constexpr (DT == XNQ_Q8_0) {
+            x = d[i] ^ 0x80808080u;
+        } else {
+            x = (d[i] >> (4 * (kg >> 1))) & 0x0F0F0F0Fu;
+            if (DT == XNQ_Q5_0 || DT == XNQ_Q5_1) x |= spread_bit4((qh >> (8 * kg + 4 * i)) & 15u);
+        }
+        q[2 * i] = magic01(x) + b;
+        q[2 * i + 1] = magic23(x) + b;
+    }
+    return h8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y};
+}
+
+__device__ __forceinline__ f4v mfma16x16x32(h8 a, h8 b) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, f4v{}, 0, 0, 0);
+}
+__device__ __forceinline__ f4v mfma16x16x16(uint2 a, uint2 b) {
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), f4v{}, 0, 0, 0);
+}
+
+template <int DT>
+__global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
+                                                                uint32_t n_tiles, float* __restrict__ y) {
+    using T = HT<DT>;
+    constexpr bool DV = true;  // the scales of planed types come with the stage (whole stages only)
+    constexpr int kSlots = 3, kWaveLds = kSlots * T::kSlot;
+    extern __shared__ __align__(16) uint8_t lds[];
+    const uint32_t total = m_tiles * n_tiles, per = (total + 7) / 8;
+    const uint32_t wi = (blockIdx.x & 7) * per + (blockIdx.x >> 3);  // one XCD: consecutive items, one column tile
+    if (wi >= total) return;
+    const uint32_t mt = wi % m_tiles, nt = wi / m_tiles;
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t col0 = nt * 32, nch = w.k / 32;
+    const uint32_t nst = (nch + 3) / 4, wst = (nst + kWaves - 1) / kWaves;
+    const uint32_t s0 = min(wave * wst, nst), s1 = min(s0 + wst, nst);
+    uint8_t* wl = lds + wave * kWaveLds;
+    const uint32_t wbase = (uint32_t)(uintptr_t)lds + wave * kWaveLds;
+    const H16Img& H = a.H;
+    const uint32_t r = lane & 15, kg = lane >> 4, rt = mt >> 1, rg = mt & 1;
+    // lanes of rows past m read the last row again (their outputs are dropped)
+    const uint32_t rl = min(r, m - 1 - mt * 16);
+    const uint32_t b_off = (kg & 1) * 1024 + (kg >> 1) * 512 + rg * 256 + rl * 16;
+    // scales and sums: the row's 8 bytes for kg == 0, else one zero entry (half 1's first)
+    const uint32_t d_off = kg == 0 ? (rg * 16 + rl) * 8 : 256;
+
+    f4v out[2], mid[2];  // the two column tiles
+#pragma unroll
+    for (int ct = 0; ct < 2; ct++) out[ct] = mid[ct] = f4v{};
+    if (s0 < s1) {
+        WOff<DT> wo;
+        weight_offsets<DT>(wo, w, col0, lane);
+        uint4 b[4];
+        uint2 bd[4], bs = make_uint2(0, 0);
+        auto load_b = [&](uint32_t st, int j) {
+            const uint32_t c = min(st * 4 + j, nch - 1);
+            b[j] = *reinterpret_cast<const uint4*>(a.h16 + ((size_t)rt * nch + c) * 2048 + b_off);
+            bd[j] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt * nch + c) * 512 + d_off);
+        };
+        auto load_s = [&](uint32_t st) {
+            if constexpr (T::kMin32)
+                bs = *reinterpret_cast<const uint2*>(a.h16 + H.s_off + ((size_t)rt * nst + st) * 512 + d_off);
+        };
+        issue_weights<DT, DV>(wo, w, s0, wbase);
+        issue_weights<DT, DV>(wo, w, min(s0 + 1, s1 - 1), wbase + T::kSlot);
+#pragma unroll
+        for (int j = 0; j < 4; j++) load_b(s0, j);
+        load_s(s0);
+        asm volatile("" ::: "memory");
+        issue_weights<DT, DV>(wo, w, min(s0 + 2, s1 - 1), wbase + 2 * T::kSlot);
+        uint32_t slot = 0;
+        for (uint32_t s = s0; s < s1; s++) {
+            const uint32_t sn = min(s + 1, s1 - 1);
+            // the DMA of stages s + 1 and s + 2 is younger than this stage's
+            wait_vm<2 * T::kND>();
+            const uint8_t* ws = wl + slot * T::kSlot;
+            // d_w (and m) of the lane's two columns, chunks 0 .. 3: operands of the
+            // rank-1 products (only lanes kg == 0 hold them)
+            uint32_t dv[2][4], mv[2][4];
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) {
+                const uint32_t c = ct * 16 + r;
+                if constexpr (T::kPlaneD) {
+                    const uint2 v = *reinterpret_cast<const uint2*>(ws + T::kNI * 1024 + c * 8);
+                    const uint32_t x = kg == 0 ? v.x : 0u, z = kg == 0 ? v.y : 0u;
+                    dv[ct][0] = x & 0xffffu; dv[ct][1] = x >> 16; dv[ct][2] = z & 0xffffu; dv[ct][3] = z >> 16;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t f = *reinterpret_cast<const uint32_t*>(ws + c * T::kSeg + j * (int)raw_stride(DT));
+                        const uint32_t v = kg == 0 && s * 4 + j < nch ? f : 0u;
+                        dv[ct][j] = v & 0xffffu;
+                        mv[ct][j] = j & 1 ? v & 0xffff0000u : v >> 16;
+                    }
+                }
+            }
+            f4v t[2];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) {
+                    uint2 wv;
+                    uint32_t qh = 0;
+                    read_chunk8<DT>(wv, qh, ws, ct * 16 + r, j, kg);
+                    const f4v I = mfma16x16x32(expand8<DT>(wv, qh, kg), as_h8(b[j]));
+                    const f4v sc = mfma16x16x16(make_uint2(dv[ct][j], 0), bd[j]);
+                    if constexpr (T::kMin32) {
+                        // per block, as the reference's vec_dot: the min and main terms cancel
+                        const f4v p = mfma16x16x16(j < 2 ? make_uint2(mv[ct][j], 0) : make_uint2(0, mv[ct][j]), bs);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            const float v = fmaf(I[e], sc[e], p[e]);
+                            t[ct][e] = j == 0 ? v : t[ct][e] + v;
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) t[ct][e] = j == 0 ? I[e] * sc[e] : fmaf(I[e], sc[e], t[ct][e]);
+                    }
+                }
+                load_b(sn, j);
+            }
+            load_s(sn);
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) mid[ct][e] += t[ct][e];
+            if ((s & 3) == 3) {
+#pragma unroll
+                for (int ct = 0; ct < 2; ct++) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) out[ct][e] += mid[ct][e];
+                    mid[ct] = f4v{};
+                }
+            }
+            // this stage's slot is read; fetch stage s + 3 into it
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            issue_weights<DT, DV>(wo, w, min(s + 3, s1 - 1), wbase + slot * T::kSlot);
+            slot = slot == 2 ? 0 : slot + 1;
+        }
+        wait_vm<0>();  // no DMA may land in the reduction below
+    }
+    // partial tiles to LDS ([wave][column tile][lane] float4), then one column
+    // tile per wavefront, summed over the eight in a tree
+    __syncthreads();
+#pragma unroll
+    for (int ct = 0; ct < 2; ct++)
+        reinterpret_cast<float4*>(lds)[(wave * 2 + ct) * 64 + lane] =
+            make_float4(out[ct][0] + mid[ct][0], out[ct][1] + mid[ct][1], out[ct][2] + mid[ct][2], out[ct][3] + mid[ct][3]);
+    __syncthreads();
+    if (wave >= 2) return;
+    float4 p[8];
+#pragma unroll
+    for (int v = 0; v < 8; v++) p[v] = reinterpret_cast<const float4*>(lds)[(v * 2 + wave) * 64 + lane];
+#pragma unroll
+    for (int d = 1; d < 8; d *= 2)
+#pragma unroll
+        for (int v = 0; v < 8; v += 2 * d) {
+            p[v].x += p[v + d].x;
+            p[v].y += p[v + d].y;
+            p[v].z += p[v + d].z;
+            p[v].w += p[v + d].w;
+        }
+    const uint32_t row = mt * 16 + r, n = col0 + wave * 16 + 4 * kg;
+    if (row >= m) return;
+    float* yr = y + (size_t)row * w.n + n;
+    if ((w.n & 3) == 0 && n + 3 < w.n) {
+        *reinterpret_cast<float4*>(yr) = p[0];
+    } else {
+        if (n < w.n) yr[0] = p[0].x;
+        if (n + 1 < w.n) yr[1] = p[0].y;
+        if (n + 2 < w.n) yr[2] = p[0].z;
+        if (n + 3 < w.n) yr[3] = p[0].w;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Prefill sizes: a workgroup owns 256 weight columns and 64 rows, K advances
 // four chunks (128) a step, and the activation tile is shared through LDS.  All
 // data moves by LDS DMA; one barrier per step publishes the shared pieces, and
@@ -892,6 +1108,18 @@ hipError_t launch_ksplit(const WView& w, const AView& a, size_t m, float* y, hip
     return hipGetLastError();
 }
 
+template <int DT>
+hipError_t launch_ksplit16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    constexpr int kWaveLds = 3 * HT<DT>::kSlot, kRed = kWaves * 2 * 64 * 16;
+    constexpr int kLds = kWaves * kWaveLds > kRed ? kWaves * kWaveLds : kRed;
+    const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_ksplit16_kernel<DT>), kLds);
+    if (e != hipSuccess) return e;
+    const uint32_t n_tiles = (w.n + 31) / 32, m_tiles = (uint32_t)((m + 15) / 16);
+    const uint32_t grid = (m_tiles * n_tiles + 7) / 8 * 8;
+    h16_ksplit16_kernel<DT><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+    return hipGetLastError();
+}
+
 template <int DT, bool DV>
 hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
     // K split over the wavefronts of a workgroup (32-row tiles up to one
@@ -904,6 +1132,14 @@ hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hip
     // of the products and about 16 us (Q5K 13): the tile pays from 148 (112)
     // tiles in every round.
     const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
+    if constexpr (!HT<DT>::kK && DV) {
+        // 16-row tiles up to one workgroup per CU (two rounds of them against one of
+        // 32-row tiles: Q8_0 N = 4096 m = 64 19.3 / 14.7), and where 32 rows would be half
+        // padding.  Not where planed scales do not come with the stage (K % 128 != 0):
+        // loads of their own inside it lose (Q8_0 1056 -> 2048 m = 48 9.1 / 8.2)
+        const size_t rt16 = (m + 15) / 16;
+        if (m <= 16 || rt16 * n32 <= 256) return launch_ksplit16<DT>(w, a, m, y, s);
+    }
     if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
     const size_t tiles = ((m + 63) / 64) * ((w.n + 255) / 256), rounds = (tiles + 255) / 256;
     if (tiles < rounds * (HT<DT>::kK ? 112 : 148)) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
