@@ -68,19 +68,19 @@ def test_super_types_ksplit(orc, dev, dt, m, k, n):
 
 
 # the 256 x 64 tile: full and ragged last tiles, K past its 16-step output sums
-@pytest.mark.parametrize("dt,m,k,n", [(dt, 640, 64, 3841) for dt in BLOCK32] + [(dt, 577, 2112, 4096) for dt in BLOCK32]
-                         + [(dt, 600, 4160, 3840) for dt in (Q4_0, Q5_1, Q8_0)])
+@pytest.mark.parametrize("dt,m,k,n", [(dt, 640, 64, 4353) for dt in BLOCK32] + [(dt, 577, 2112, 4608) for dt in BLOCK32]
+                         + [(dt, 600, 4160, 4352) for dt in (Q4_0, Q5_1, Q8_0)])
 def test_block_types_tile(orc, dev, dt, m, k, n):
     check(orc, dev, dt, m, k, n, 400 + dt + m)
 
 
 @pytest.mark.parametrize("dt", [Q4_0, Q8_0])
 def test_block_types_tile_odd_blocks(orc, dev, dt):
-    check(orc, dev, dt, 600, 1056, 3842, 500 + dt)
+    check(orc, dev, dt, 600, 1056, 4354, 500 + dt)
 
 
 @pytest.mark.parametrize("dt", SUPER)
-@pytest.mark.parametrize("m,k,n", [(512, 256, 3585), (449, 1280, 4096)])
+@pytest.mark.parametrize("m,k,n", [(512, 256, 4353), (449, 1280, 4352), (520, 4352, 4096)])
 def test_super_types_tile(orc, dev, dt, m, k, n):
     check(orc, dev, dt, m, k, n, 600 + dt + m)
 

@@ -26,8 +26,9 @@
 // two K = 16 steps.
 //
 // Summation.  Long chains of f32 additions are split so that the rounding
-// error stays at the level of the matvec kernels' lane tree: four blocks,
-// then four stages, then the rest, then (wavefronts that split K) a tree.
+// error stays at or below that of the matvec kernels' lane tree: four blocks,
+// then four stages, then the rest; super-blocks in eights.  Wavefronts that
+// split K, and the stores of a long K, are added in 64 bits.
 #include <type_traits>
 
 #include "xnq_device.h"
@@ -356,9 +357,26 @@ __device__ __forceinline__ void super_unit(const f16v& I, const Scales<DT>& S, c
 // still puts two wavefronts on every SIMD.  Each wavefront streams its share of
 // the weights through its own LDS ring (LDS DMA in whole cache lines, two
 // stages ahead) and its share of the activation image straight into registers
-// (a stage ahead); there is no barrier until the eight partial tiles are added,
-// in a tree, through LDS.
+// (a stage ahead); there is no barrier until the eight partial tiles are added
+// through LDS.
 // ---------------------------------------------------------------------------
+// The eight wavefronts' partials of four outputs, added in 64 bits: one rounding
+// for the eight, which pays for those of the longer chains over a wavefront's
+// stages (relative L2 error against exact sums, the matvec kernels' / these, Q8_0: K = 1024
+// 6.6e-8 / 4.7e-8, 4096 7.4e-8 / 6.3e-8, 14336 8.4e-8 / 7.4e-8).
+__device__ __forceinline__ float4 sum_waves(const float4* p, int stride) {
+    double x = 0, y = 0, z = 0, w = 0;
+#pragma unroll
+    for (int v = 0; v < kWaves; v++) {
+        const float4 q = p[v * stride];
+        x += q.x;
+        y += q.y;
+        z += q.z;
+        w += q.w;
+    }
+    return make_float4((float)x, (float)y, (float)z, (float)w);
+}
+
 template <int DT, int TM, bool DV>
 __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
                                                               uint32_t n_tiles, float* __restrict__ y) {
@@ -508,7 +526,7 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
         wait_vm<0>();  // no DMA may land in the reduction below
     }
     // partial tiles to LDS ([wave][tile, quad][lane] float4), then one quad of
-    // one tile per wavefront, summed over the eight in a tree
+    // one tile per wavefront, summed over the eight
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TM; i++)
@@ -523,28 +541,17 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
         }
     __syncthreads();
     for (uint32_t iq = wave; iq < TM * 4; iq += kWaves) {
-        float4 p[8];
-#pragma unroll
-        for (int v = 0; v < 8; v++) p[v] = reinterpret_cast<const float4*>(lds)[(v * (TM * 4) + iq) * 64 + lane];
-#pragma unroll
-        for (int d = 1; d < 8; d *= 2)
-#pragma unroll
-            for (int v = 0; v < 8; v += 2 * d) {
-                p[v].x += p[v + d].x;
-                p[v].y += p[v + d].y;
-                p[v].z += p[v + d].z;
-                p[v].w += p[v + d].w;
-            }
+        const float4 o = sum_waves(reinterpret_cast<const float4*>(lds) + iq * 64 + lane, TM * 4 * 64);
         const uint32_t row = (mt * TM + (iq >> 2)) * 32 + lrow, n = col0 + 8 * (iq & 3) + 4 * g;
         if (row >= m) continue;
         float* yr = y + (size_t)row * w.n + n;
         if ((w.n & 3) == 0 && n + 3 < w.n) {
-            *reinterpret_cast<float4*>(yr) = p[0];
+            *reinterpret_cast<float4*>(yr) = o;
         } else {
-            if (n < w.n) yr[0] = p[0].x;
-            if (n + 1 < w.n) yr[1] = p[0].y;
-            if (n + 2 < w.n) yr[2] = p[0].z;
-            if (n + 3 < w.n) yr[3] = p[0].w;
+            if (n < w.n) yr[0] = o.x;
+            if (n + 1 < w.n) yr[1] = o.y;
+            if (n + 2 < w.n) yr[2] = o.z;
+            if (n + 3 < w.n) yr[3] = o.w;
         }
     }
 }
@@ -732,7 +739,7 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a
         wait_vm<0>();  // no DMA may land in the reduction below
     }
     // partial tiles to LDS ([wave][column tile][lane] float4), then one column
-    // tile per wavefront, summed over the eight in a tree
+    // tile per wavefront, summed over the eight
     __syncthreads();
 #pragma unroll
     for (int ct = 0; ct < 2; ct++)
@@ -740,28 +747,17 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a
             make_float4(out[ct][0] + mid[ct][0], out[ct][1] + mid[ct][1], out[ct][2] + mid[ct][2], out[ct][3] + mid[ct][3]);
     __syncthreads();
     if (wave >= 2) return;
-    float4 p[8];
-#pragma unroll
-    for (int v = 0; v < 8; v++) p[v] = reinterpret_cast<const float4*>(lds)[(v * 2 + wave) * 64 + lane];
-#pragma unroll
-    for (int d = 1; d < 8; d *= 2)
-#pragma unroll
-        for (int v = 0; v < 8; v += 2 * d) {
-            p[v].x += p[v + d].x;
-            p[v].y += p[v + d].y;
-            p[v].z += p[v + d].z;
-            p[v].w += p[v + d].w;
-        }
+    const float4 o = sum_waves(reinterpret_cast<const float4*>(lds) + wave * 64 + lane, 2 * 64);
     const uint32_t row = mt * 16 + r, n = col0 + wave * 16 + 4 * kg;
     if (row >= m) return;
     float* yr = y + (size_t)row * w.n + n;
     if ((w.n & 3) == 0 && n + 3 < w.n) {
-        *reinterpret_cast<float4*>(yr) = p[0];
+        *reinterpret_cast<float4*>(yr) = o;
     } else {
-        if (n < w.n) yr[0] = p[0].x;
-        if (n + 1 < w.n) yr[1] = p[0].y;
-        if (n + 2 < w.n) yr[2] = p[0].z;
-        if (n + 3 < w.n) yr[3] = p[0].w;
+        if (n < w.n) yr[0] = o.x;
+        if (n + 1 < w.n) yr[1] = o.y;
+        if (n + 2 < w.n) yr[2] = o.z;
+        if (n + 3 < w.n) yr[3] = o.w;
     }
 }
 
@@ -830,7 +826,9 @@ __global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView
         issue_weights<DT, true>(wo, w, min(sb, nsb - 1), lbase + wls + slot * T::kSlot);
     };
 
-    f16v out[2], I[2];
+    // two levels of sums, eight super-blocks each in the first: one chain over a long
+    // K rounds off more than the matvec's lanes do
+    f16v out[2], mid[2], I[2];
 #pragma unroll
     for (int i = 0; i < 2; i++) out[i] = f16v{};
     issue_b(0, 0);
@@ -840,55 +838,63 @@ __global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView
     uint32_t slot = 0, free_slot = 2;
     Scales<DT> S;
     uint8_t* dl = lds + Y::kOffDl + wave * T::kDl;
-    for (uint32_t sb = 0; sb < nsb; sb++) {
-        const uint8_t* ws = lds + wls + (sb & 1) * T::kSlot;
-        const uint8_t* sbp = lds + Y::kOffSb + (sb & 1) * Y::kSb;
+    for (uint32_t sb8 = 0; sb8 < nsb; sb8 += 8) {
+        const uint32_t e8 = min(sb8 + 8, nsb);
+        mid[0] = mid[1] = f16v{};
+        for (uint32_t sb = sb8; sb < e8; sb++) {
+            const uint8_t* ws = lds + wls + (sb & 1) * T::kSlot;
+            const uint8_t* sbp = lds + Y::kOffSb + (sb & 1) * Y::kSb;
 #pragma unroll
-        for (int p = 0; p < 2; p++) {
-            // this step has landed, and every wavefront is past the previous one.  Younger
-            // than its DMA: at the first step the next step's tile, at the second also the
-            // next super-block's pieces
-            if (p == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB) : "memory");
-            else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB + Y::kNSb + T::kND) : "memory");
-            issue_b(2 * sb + p + 2, free_slot);
-            if (p == 0) {
-                issue_sb(sb + 1, (sb + 1) & 1);
-                issue_w(sb + 1, (sb + 1) & 1);
-                read_scales<DT, true>(S, w, ws, dl, col0, lane, sb, nch);
-            }
-            const uint8_t* bs = lds + slot * Y::kBSlot + lane * 16;
-#pragma unroll
-            for (int jj = 0; jj < 4; jj++) {
-                const int j = 4 * p + jj;
-                h8 A[2];
-                Bytes by;
-                read_chunk<DT>(by, ws, lrow, j, g);
-                expand<DT>(by, j, g, S.hd, A);
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    const uint4 b0 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048);
-                    const uint4 b1 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048 + 1024);
-                    I[i] = mfma16(A[0], as_h8(b0), j == 0 ? f16v{} : I[i]);
-                    I[i] = mfma16(A[1], as_h8(b1), I[i]);
+            for (int p = 0; p < 2; p++) {
+                // this step has landed, and every wavefront is past the previous one.  Younger
+                // than its DMA: at the first step the next step's tile, at the second also the
+                // next super-block's pieces
+                if (p == 0) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB) : "memory");
+                else asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(Y::kNB + Y::kNSb + T::kND) : "memory");
+                issue_b(2 * sb + p + 2, free_slot);
+                if (p == 0) {
+                    issue_sb(sb + 1, (sb + 1) & 1);
+                    issue_w(sb + 1, (sb + 1) & 1);
+                    read_scales<DT, true>(S, w, ws, dl, col0, lane, sb, nch);
                 }
+                const uint8_t* bs = lds + slot * Y::kBSlot + lane * 16;
+#pragma unroll
+                for (int jj = 0; jj < 4; jj++) {
+                    const int j = 4 * p + jj;
+                    h8 A[2];
+                    Bytes by;
+                    read_chunk<DT>(by, ws, lrow, j, g);
+                    expand<DT>(by, j, g, S.hd, A);
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const uint4 b0 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048);
+                        const uint4 b1 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048 + 1024);
+                        I[i] = mfma16(A[0], as_h8(b0), j == 0 ? f16v{} : I[i]);
+                        I[i] = mfma16(A[1], as_h8(b1), I[i]);
+                    }
+                }
+                free_slot = slot;
+                slot = slot == 2 ? 0 : slot + 1;
             }
-            free_slot = slot;
-            slot = slot == 2 ? 0 : slot + 1;
-        }
-        float dw[16], dm[16];
-        const float* dp = reinterpret_cast<const float*>(dl) + 4 * g;
+            float dw[16], dm[16];
+            const float* dp = reinterpret_cast<const float*>(dl) + 4 * g;
 #pragma unroll
-        for (int e = 0; e < 16; e++) {
-            dw[e] = dp[8 * (e >> 2) + (e & 3)];
-            if (T::kMinK) dm[e] = dp[32 + 8 * (e >> 2) + (e & 3)];
+            for (int e = 0; e < 16; e++) {
+                dw[e] = dp[8 * (e >> 2) + (e & 3)];
+                if (T::kMinK) dm[e] = dp[32 + 8 * (e >> 2) + (e & 3)];
+            }
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const float da = reinterpret_cast<const float*>(sbp)[i * 32 + lrow];
+                uint4 ms = make_uint4(0, 0, 0, 0);
+                if constexpr (T::kMinK) ms = *reinterpret_cast<const uint4*>(sbp + 256 + i * 1024 + lane * 16);
+                super_unit<DT>(I[i], S, ms, da, dw, dm, mid[i]);
+            }
         }
 #pragma unroll
-        for (int i = 0; i < 2; i++) {
-            const float da = reinterpret_cast<const float*>(sbp)[i * 32 + lrow];
-            uint4 ms = make_uint4(0, 0, 0, 0);
-            if constexpr (T::kMinK) ms = *reinterpret_cast<const uint4*>(sbp + 256 + i * 1024 + lane * 16);
-            super_unit<DT>(I[i], S, ms, da, dw, dm, out[i]);
-        }
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int e = 0; e < 16; e++) out[i][e] += mid[i][e];
     }
     wait_vm<0>();  // no DMA outlives the workgroup's LDS
     const uint32_t nb0 = col0 + 4 * g;
@@ -999,8 +1005,10 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
 
     f16v out, mid;
 
-    // The output tile, stored (first) or added to.  Long K adds to it every 16
-    // steps: a last level of the sum that needs no registers.
+    // The output tile, out + mid, stored (first) or added to.  Long K adds to it
+    // every 16 steps: a last level of the sum that needs no registers.  It is added in
+    // 64 bits, one rounding for the two sums.
+    auto add3 = [](float z, float o, float t) { return (float)((double)z + (double)o + (double)t); };
     auto flush = [&](bool first) __attribute__((always_inline)) {
         uint32_t r0 = lrow;
         asm volatile("" : "+v"(r0));  // keeps the addresses out of the step loop's registers
@@ -1011,17 +1019,20 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
             for (int q = 0; q < 4; q++) {
                 const uint32_t n = col0 + 4 * g + 8 * q;
                 if (n + 3 < w.n && (w.n & 3) == 0) {
-                    float4 o = make_float4(out[4 * q], out[4 * q + 1], out[4 * q + 2], out[4 * q + 3]);
+                    float4 o = make_float4(out[4 * q] + mid[4 * q], out[4 * q + 1] + mid[4 * q + 1], out[4 * q + 2] + mid[4 * q + 2],
+                                           out[4 * q + 3] + mid[4 * q + 3]);
                     float4* p = reinterpret_cast<float4*>(yr + n);
                     if (!first) {
                         const float4 z = *p;
-                        o = make_float4(o.x + z.x, o.y + z.y, o.z + z.z, o.w + z.w);
+                        o = make_float4(add3(z.x, out[4 * q], mid[4 * q]), add3(z.y, out[4 * q + 1], mid[4 * q + 1]),
+                                        add3(z.z, out[4 * q + 2], mid[4 * q + 2]), add3(z.w, out[4 * q + 3], mid[4 * q + 3]));
                     }
                     *p = o;
                 } else {
 #pragma unroll
                     for (int e = 0; e < 4; e++)
-                        if (n + e < w.n) yr[n + e] = first ? out[4 * q + e] : yr[n + e] + out[4 * q + e];
+                        if (n + e < w.n)
+                            yr[n + e] = first ? out[4 * q + e] + mid[4 * q + e] : add3(yr[n + e], out[4 * q + e], mid[4 * q + e]);
                 }
             }
         }
@@ -1080,13 +1091,23 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
         for (int e = 0; e < 16; e++) mid[e] += t[e];
         slot = slot + 1 == Y::kSlots ? 0 : slot + 1;
     };
-    for (uint32_t s16 = 0; s16 < nstep; s16 += 16) {
-        const uint32_t e16 = min(s16 + 16, nstep);
+    // Steps summed in mid, and between two stores of the tile (even shares of at most 16).
+    // So the relative L2 error against exact sums is no larger than the matvec kernels',
+    // theirs / this: Q4_0 K = 1024 6.6e-8 / 6.3e-8, 2560 7.2e-8 / 6.9e-8, 4096 7.4e-8 /
+    // 7.3e-8, 14336 8.4e-8 / 8.3e-8.  Q4_1's has one rounding a block more to make up
+    // for, which takes shorter chains over a short K (7.65e-8 / 7.54e-8 at 4096 with,
+    // 7.71e-8 without; 348 against 325 us at m = 512 4096 -> 14336).
+    const uint32_t fold = DT == XNQ_Q4_1 && nstep < 24 ? 2 : 4;
+    const uint32_t most = DT == XNQ_Q4_1 && nstep <= 40 ? 2 * fold : 16, stores = (nstep + most - 1) / most;
+    const uint32_t share = (nstep + stores * fold - 1) / (stores * fold) * fold;
+    for (uint32_t s16 = 0; s16 < nstep; s16 += share) {
+        const uint32_t e16 = min(s16 + share, nstep);
         out = f16v{};
-        for (uint32_t s4 = s16; s4 < e16; s4 += 4) {
-            const uint32_t e4 = min(s4 + 4, e16);
+        for (uint32_t s4 = s16; s4 < e16; s4 += fold) {
+            const uint32_t e4 = min(s4 + fold, e16);
             mid = f16v{};
             for (uint32_t s = s4; s < e4; s++) step(s);
+            if (e4 == e16) break;
 #pragma unroll
             for (int e = 0; e < 16; e++) out[e] += mid[e];
         }
@@ -1122,15 +1143,6 @@ hipError_t launch_ksplit16(const WView& w, const AView& a, size_t m, float* y, h
 
 template <int DT, bool DV>
 hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
-    // K split over the wavefronts of a workgroup (32-row tiles up to one
-    // workgroup per CU, then 64-row tiles) against the 256 x 64 tile, us, graph
-    // steps, K = 4096, Q8_0: N = 1024 m = 256 17.1 / 21.3 / 76, 512 30.5 / 24.6 / 79;
-    // N = 4096 m = 64 15.2 / 19.1 / 73, 128 24.8 / 20.9 / 74, 512 88 / 65 / 77;
-    // N = 14336 m = 128 77 / 67 / 81, 256 146 / 111 / 85.  Q5K: 6144 m = 64 22.7 / 18.1 /
-    // 47, 256 57 / 43 / 50, 512 120 / 83 / 55.  A round of tiles (one per CU) costs the
-    // same however few it holds, a round of 64-row K-split workgroups an eighth
-    // of the products and about 16 us (Q5K 13): the tile pays from 148 (112)
-    // tiles in every round.
     const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
     if constexpr (!HT<DT>::kK && DV) {
         // 16-row tiles up to one workgroup per CU (two rounds of them against one of
@@ -1140,9 +1152,19 @@ hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hip
         const size_t rt16 = (m + 15) / 16;
         if (m <= 16 || rt16 * n32 <= 256) return launch_ksplit16<DT>(w, a, m, y, s);
     }
+    // 32-row tiles up to one workgroup per CU, then 64-row tiles (Q8_0, K = 4096, us, graph
+    // steps: N = 1024 m = 256 17 / 21, 512 31 / 25; N = 4096 m = 64 15 / 19, 128 25 / 21)
     if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
+    // A round of 256 x 64 tiles (one a CU) costs the same however few it holds; a round
+    // of 64-row K-split workgroups is the products of 32 tiles.  So the tile pays from
+    // so many K-split rounds, us, K = N = 4096, K-split / tile: Q2K m = 256 (2 rounds)
+    // 40 / 52, 320 (3) 59 / 52; Q5K 384 (3) 46 / 52, 448 (4) 58 / 52; Q3K 384 42 / 52,
+    // 512 (4) 54 / 52; Q8_0 512 (4) 66 / 67, 576 (5) 81 / 68; Q4_0 512 65 / 70, 576
+    // 79 / 70; Q4_1 512 140 / 141, 576 169 / 146; Q5_0 640 (5) 80 / 92, 768 (6) 97 / 93;
+    // Q5_1 640 133 / 135, 768 163 / 142; scales not staged (Q8_0, K = 4160) 640 88 / 103.
+    constexpr size_t kRounds = DT == XNQ_Q2K ? 2 : DT == XNQ_Q5K ? 3 : DT == XNQ_Q5_0 || DT == XNQ_Q5_1 || !DV ? 5 : 4;
     const size_t tiles = ((m + 63) / 64) * ((w.n + 255) / 256), rounds = (tiles + 255) / 256;
-    if (tiles < rounds * (HT<DT>::kK ? 112 : 148)) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
+    if (tiles <= rounds * kRounds * 32) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
     const uint32_t m_tiles = (uint32_t)((m + 63) / 64), n_tiles = (w.n + 255) / 256, grid = (m_tiles * n_tiles + 7) / 8 * 8;
     if constexpr (HT<DT>::kK) {
         constexpr int kLds = TLay<DT>::kLds;
