@@ -276,9 +276,9 @@ static bool tiled_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
 // type, m and K only.  K is bounded as for the matvec kernels, whose LDS holds
 // a row image.  The matvec kernels take up to 8 rows in one launch and read
 // the weights again for every further 8; the f16 kernels cost the same from 1
-// to 32 rows.  m = 8 and 16, K = 4096, us, matvec / f16: Q8_0 N = 1024 8.0 / 12.7
-// and 13.2 / 12.7, 14336 22.3 / 28.0 and 41.7 / 28.5; Q4_0 14336 22.8 / 23.5 and
-// 42.7 / 23.5; Q5K 6144 14.1 / 13.7 and 24.5 / 13.8.
+// to 16 (32-element types) or 32 rows.  m = 8 (f16: 9) and 16, K = 4096, us, matvec / f16:
+// Q8_0 N = 1024 8.0 / 11.3 and 13.2 / 11.3, 14336 22.3 / 26.2 and 41.7 / 26.4; Q4_0
+// 14336 22.8 / 22.3 and 42.7 / 22.4; Q5K 6144 14.1 / 13.7 and 24.5 / 13.8.
 static bool h16_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
     return forced == 0 && m > 8 && h16_supported(weight_dtype) &&
            act_img((uint32_t)k, is_kquant(weight_dtype)).row_bytes <= 160 * 1024;
