@@ -92,6 +92,49 @@ def test_subnormal_scales(orc, dev, dt, wscale, xscale):
     check(orc, dev, dt, 40, 1024, 64, 700 + dt, wscale, xscale)
 
 
+def check_nonfinite(got, want, m):
+    """NaN and either infinity where the matvec kernels have them; rows without
+    them within 32-bit sums."""
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    assert np.array_equal(np.isposinf(got), np.isposinf(want)) and np.array_equal(np.isneginf(got), np.isneginf(want))
+    ok = np.isfinite(want).all(axis=1)
+    assert ok.sum() >= m - 8
+    err = np.linalg.norm(got[ok].astype(np.float64) - want[ok]) / np.linalg.norm(want[ok].astype(np.float64))
+    assert err < 2e-6
+
+
+def run_both(orc, dev, dt, m, k, n, x, seed):
+    """(matmul_t, the matvec kernels') of random weights on x."""
+    from xn_amd.quantized import set_route
+
+    blocks = orc.from_float(dt, np.random.default_rng(seed).normal(0, 0.02, (n, k)).astype(np.float32))
+    qt = upload(blocks, n, k, dt, dev)
+    got = run(qt, x, m, k, n, dev)
+    try:
+        set_route(1)
+        return got, run(qt, x, m, k, n, dev)
+    finally:
+        set_route(0)
+
+
+# (m, n): 16-row tiles, one and two 32-row tiles of the K-split kernel, the 256 x 64 tile
+NONFINITE_TILES = [(40, 64), (64, 4096), (64, 8224), (600, 4352)]
+
+
+@pytest.mark.parametrize("dt", [Q4_1, Q5_1])
+@pytest.mark.parametrize("m,n", NONFINITE_TILES)
+def test_overflowing_block_sums(orc, dev, dt, m, n):
+    """A Q8_1 sum past the f16 range beside a finite scale, alone in its stage of
+    four blocks, beside one of the other sign, and from a single large element."""
+    k = 320
+    x = np.random.default_rng(850 + dt).normal(0, 1, (m, k)).astype(np.float32)
+    x[3, 64:96], x[5, 128:160], x[7, 40], x[9, 288:] = 3000.0, -3000.0, 7e4, 2500.0
+    x[11, 0:32], x[11, 96:128] = 3000.0, -3000.0
+    got, want = run_both(orc, dev, dt, m, k, n, x, 850 + dt)
+    assert np.isinf(want[[3, 5, 7, 9]]).any(axis=1).all()
+    check_nonfinite(got, want, m)
+
+
 @pytest.mark.parametrize("dt", [Q4_0, Q4_1, Q8_0, Q2K, Q5K])
 @pytest.mark.parametrize("m,n", [(40, 64), (600, 3840)])
 def test_nonfinite_rows(orc, dev, dt, m, n):

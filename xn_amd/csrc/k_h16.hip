@@ -239,7 +239,7 @@ template <int DT>
 struct Scales {
     uint4 hd;                            // K types: the block header's words
     uint2 d[HT<DT>::kK ? 1 : 4];      // 32-element types: operand of the scale product, chunk j
-    uint2 m[HT<DT>::kMin32 ? 4 : 1];  // and of the min product (the chunk's K slot only)
+    uint2 m[HT<DT>::kMin32 ? 4 : 1];  // and of the min product
     uint4 mn;                            // K types: min-term operand
 };
 
@@ -297,16 +297,21 @@ __device__ __forceinline__ void read_scales(Scales<DT>& S, const WView& w, const
                 const uint32_t f = *reinterpret_cast<const uint32_t*>(col + j * (int)raw_stride(DT));
                 const bool live = st * 4 + j < nch;
                 dv[j] = live ? f & 0xffffu : 0u;
-                if constexpr (T::kMin32) {
-                    const uint32_t mv = live && h == 0 ? f >> 16 : 0u;
-                    const uint32_t v = j & 1 ? mv << 16 : mv;
-                    S.m[j] = j < 2 ? make_uint2(v, 0) : make_uint2(0, v);
-                }
+                if constexpr (T::kMin32) S.m[j] = make_uint2(live && h == 0 ? f >> 16 : 0u, 0);
             }
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) S.d[j] = make_uint2(h == 0 ? dv[j] : 0u, 0);
     }
+}
+
+// Operand B of chunk j's min product out of a stage's four f16 sums: the other
+// three stay out of it also where the weight operand is zero, since a sum that
+// overflowed f16 (a block's sum past 65504, its scale still finite) would make
+// them 0 x inf = NaN.
+__device__ __forceinline__ uint2 chunk_sum(const uint2& s, int j) {
+    const uint32_t v = j < 2 ? s.x : s.y;
+    return make_uint2(j & 1 ? v >> 16 : v & 0xffffu, 0);
 }
 
 // One 32 x 32 unit (a chunk of a 32-element type by a row tile): the matrix
@@ -321,7 +326,7 @@ __device__ __forceinline__ void unit_mma(Unit<DT>& u, const h8* a, const Scales<
     u.I = mfma16(a[0], as_h8(b[0]), f16v{});
     u.sc = mfma8(S.d[j], bd);
     u.I = mfma16(a[1], as_h8(b[1]), u.I);
-    if constexpr (HT<DT>::kMin32) u.p = mfma8(S.m[j], bs);
+    if constexpr (HT<DT>::kMin32) u.p = mfma8(S.m[j], chunk_sum(bs, j));
 }
 template <int DT>
 __device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t) {
@@ -689,7 +694,7 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a
                         const uint32_t f = *reinterpret_cast<const uint32_t*>(ws + c * T::kSeg + j * (int)raw_stride(DT));
                         const uint32_t v = kg == 0 && s * 4 + j < nch ? f : 0u;
                         dv[ct][j] = v & 0xffffu;
-                        mv[ct][j] = j & 1 ? v & 0xffff0000u : v >> 16;
+                        mv[ct][j] = v >> 16;
                     }
                 }
             }
@@ -705,7 +710,7 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a
                     const f4v sc = mfma16x16x16(make_uint2(dv[ct][j], 0), bd[j]);
                     if constexpr (T::kMin32) {
                         // per block, as the reference's vec_dot: the min and main terms cancel
-                        const f4v p = mfma16x16x16(j < 2 ? make_uint2(mv[ct][j], 0) : make_uint2(0, mv[ct][j]), bs);
+                        const f4v p = mfma16x16x16(make_uint2(mv[ct][j], 0), chunk_sum(bs, j));
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
                             const float v = fmaf(I[e], sc[e], p[e]);
