@@ -127,11 +127,24 @@ def test_overflowing_block_sums(orc, dev, dt, m, n):
     """A Q8_1 sum past the f16 range beside a finite scale, alone in its stage of
     four blocks, beside one of the other sign, and from a single large element."""
     k = 320
-    x = np.random.default_rng(850 + dt).normal(0, 1, (m, k)).astype(np.float32)
+    x = np.random.default_rng(5850 + dt).normal(0, 1, (m, k)).astype(np.float32)
     x[3, 64:96], x[5, 128:160], x[7, 40], x[9, 288:] = 3000.0, -3000.0, 7e4, 2500.0
     x[11, 0:32], x[11, 96:128] = 3000.0, -3000.0
     got, want = run_both(orc, dev, dt, m, k, n, x, 850 + dt)
     assert np.isinf(want[[3, 5, 7, 9]]).any(axis=1).all()
+    check_nonfinite(got, want, m)
+
+
+@pytest.mark.parametrize("dt,k", [(Q8_0, 1056), (Q4_0, 160), (Q4_1, 576), (Q5_0, 576), (Q5_1, 320)])
+@pytest.mark.parametrize("m,n", NONFINITE_TILES)
+def test_overflowing_scale_in_a_cut_stage(orc, dev, dt, k, m, n):
+    """An infinite activation scale in the last block of a K that is not whole
+    stages of four blocks: the blocks that fill the stage up add nothing."""
+    x = np.random.default_rng(5870 + dt).normal(0, 1, (m, k)).astype(np.float32)
+    x[3, -5], x[5, k - 32] = 1e9, -1e9
+    got, want = run_both(orc, dev, dt, m, k, n, x, 870 + dt)
+    if dt not in (Q4_1, Q5_1):  # (their infinite sum times m meets the infinite product)
+        assert np.isinf(want[[3, 5]]).any(axis=1).all()
     check_nonfinite(got, want, m)
 
 

@@ -112,7 +112,8 @@ __device__ __forceinline__ void weight_offsets(WOff<DT>& o, const WView& w, uint
 }
 
 // DMA of stage st into the LDS slot at byte address `to`.  A stage past the end of the row
-// (K not a multiple of 128) re-reads the row's last piece; its scales are zeroed.
+// (K not a multiple of 128) re-reads the row's last piece; its scales are zeroed, as are the
+// activation's for those chunks in the image (an infinite one would make them NaN).
 template <int DT, bool DV>
 __device__ __forceinline__ void issue_weights(const WOff<DT>& o, const WView& w, uint32_t st, uint32_t to) {
     using T = HT<DT>;
@@ -430,12 +431,12 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
         uint2 bs32[TM];  // Q4_1, Q5_1: min-term operand of the stage
         auto load_unit = [&](uint32_t st, int u, int slot) {
             const int j = u / TM, i = u % TM;
-            const uint32_t c = min(st * T::kCH + j, nch - 1);
+            const uint32_t cj = st * T::kCH + j, c = min(cj, nch - 1);
             const uint8_t* p = a.h16 + ((size_t)rt[i] * nch + c) * 2048 + bl[i] * 16;
             b[slot][0] = *reinterpret_cast<const uint4*>(p);
             b[slot][1] = *reinterpret_cast<const uint4*>(p + 1024);
             if constexpr (!T::kK)
-                bd[slot] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt[i] * nch + c) * 512 + lane * 8);
+                bd[slot] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt[i] * nst * 4 + cj) * 512 + lane * 8);
         };
         auto load_scales = [&](uint32_t st) {
 #pragma unroll
@@ -657,9 +658,9 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit16_kernel(WView w, AView a
         uint4 b[4];
         uint2 bd[4], bs = make_uint2(0, 0);
         auto load_b = [&](uint32_t st, int j) {
-            const uint32_t c = min(st * 4 + j, nch - 1);
+            const uint32_t cj = st * 4 + j, c = min(cj, nch - 1);
             b[j] = *reinterpret_cast<const uint4*>(a.h16 + ((size_t)rt * nch + c) * 2048 + b_off);
-            bd[j] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt * nch + c) * 512 + d_off);
+            bd[j] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt * nst * 4 + cj) * 512 + d_off);
         };
         auto load_s = [&](uint32_t st) {
             if constexpr (T::kMin32)
@@ -985,14 +986,14 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
     // scales from wavefronts 0 .. 3, the sums from 4, a column group's weights
     // from its two wavefronts in turn
     const uint8_t* const b0 = a.h16 + (size_t)(rh ? rt1 : rt0) * nch * 2048 + (cw & 1) * 1024;
-    const uint8_t* const d0 = a.h16 + H.d_off + (size_t)(wave >> 1 ? rt1 : rt0) * nch * 512;
+    const uint8_t* const d0 = a.h16 + H.d_off + (size_t)(wave >> 1 ? rt1 : rt0) * nstep * 2048;
     const uint8_t* const s0 = a.h16 + H.s_off + (size_t)rt0 * nstep * 512;
     auto issue = [&](uint32_t q, uint32_t slot) {
         const uint32_t to = lbase + slot * Y::kBSlot, tw = lbase + Y::kOffW + slot * Y::kWSlot + cw * T::kSlot;
         const uint32_t qc = min(q, nstep - 1);
         dma16(b0 + (size_t)min(qc * 4 + (cw >> 1), nch - 1) * 2048, lane * 16, to + wave * 1024);
         if (wave < 4)
-            dma16(d0, min(qc * 4 + 2 * (wave & 1) + g, nch - 1) * 512 + lrow * 16, to + Y::kSc + wave * 1024);
+            dma16(d0, (qc * 4 + 2 * (wave & 1) + g) * 512 + lrow * 16, to + Y::kSc + wave * 1024);
         if (T::kMin32 && wave == 4) dma16(s0 + qc * 512, (g ? (rt1 - rt0) * nstep * 512 : 0u) + lrow * 16, to + Y::kMs);
 #pragma unroll
         for (int i = 0; i < T::kNI; i++) {

@@ -188,8 +188,8 @@ __global__ __launch_bounds__(256) void quantize_q80_h16_kernel(const float* __re
     *reinterpret_cast<uint2*>(sq[wave] + (((sub >> 1) & 1) * 2 + (sub >> 2)) * 128 + rr * 16 + (sub & 1) * 8) =
         quants_f16(r.packed);
     const size_t rt = grp / 4, r32 = (grp & 3) * 8 + rr;
-    if (live && sub < 2)
-        reinterpret_cast<uint2*>(img + H.d_off)[(rt * nch + c) * 64 + sub * 32 + r32] = make_uint2(sub == 0 ? r.dh : 0u, 0u);
+    if (sub < 2)  // (chunks past the end: zeros)
+        reinterpret_cast<uint2*>(img + H.d_off)[(rt * nst * 4 + c) * 64 + sub * 32 + r32] = make_uint2(sub == 0 ? r.dh : 0u, 0u);
     if (mins && sub < 2) {
         const uint16_t s = f32_to_f16_bits(f16_bits_to_f32(f32_to_f16_bits((float)r.sum)) * f16_bits_to_f32(r.dh));
         reinterpret_cast<uint16_t*>(img + H.s_off)[((rt * nst + st) * 64 + sub * 32 + r32) * 4 + wave] =

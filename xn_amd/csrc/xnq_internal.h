@@ -153,7 +153,8 @@ __host__ __device__ inline TileImg tile_img(size_t m, uint32_t k) {
 //   quants  [tile][chunk c][step 2][lane 64][16]: elements 16 half + 8 step ..
 //           + 7 of the chunk as f16 whole numbers
 //   32-element activations (Q8_0 / Q8_1 blocks), nst = ceil(nch / 4):
-//     d     [tile][chunk][lane 64][8]: {f16 scale, 0, 0, 0} for half 0, zeros for half 1
+//     d     [tile][chunk < 4 nst][lane 64][8]: {f16 scale, 0, 0, 0} for half 0, zeros
+//           for half 1 and for the chunks past nch of the last stage
 //     s     [tile][4-chunk stage][lane 64][8] (Q4_1, Q5_1 only): Q8_1's f16 s of the
 //           stage's four chunks for half 0, 0 for half 1
 //   Q8K activations:
@@ -169,7 +170,7 @@ __host__ __device__ inline H16Img h16_img(size_t m, uint32_t k, bool kquant, boo
     H.rts = (uint32_t)((m + 31) / 32);
     const size_t nch = k / 32, nst = (nch + 3) / 4;
     H.d_off = H.rts * nch * 2048;
-    H.s_off = H.d_off + (kquant ? H.rts * (nch / 8) * 128 : H.rts * nch * 512);
+    H.s_off = H.d_off + (kquant ? H.rts * (nch / 8) * 128 : H.rts * nst * 2048);
     H.bytes = H.s_off + (kquant ? H.rts * (nch / 8) * 1024 : mins32 ? H.rts * nst * 512 : 0);
     return H;
 }
