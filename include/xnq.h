@@ -195,7 +195,13 @@ xnq_status xnq_mlp_t(const xnq_qtensor* gate, const xnq_qtensor* up, const xnq_q
  * quantize_lhs writes (the quantized activation image);
  * xnq_qtensor_workspace_size adds the scratch matmul_preq may use on this
  * weight (split-K partial sums of the MFMA route).  matmul_preq is told the
- * workspace's size and uses no scratch it does not fit. */
+ * workspace's size and uses no scratch it does not fit.
+ *
+ * A Q4_K or Q6_K weight takes a workspace that quantize_lhs wrote for its own
+ * dtype and the same m and k.  A weight of the other dtypes takes one written
+ * for any dtype of the same activation blocks (Q8_0: Q8_0, Q4_0, Q4_1, Q5_0,
+ * Q5_1; Q8_K: Q2K, Q3K, Q4K, Q5K, Q6K) with the same k and at least m rows,
+ * uses the first m of them, and only reads it. */
 size_t xnq_lhs_workspace_size(uint32_t weight_dtype, size_t m, size_t k);
 size_t xnq_qtensor_workspace_size(const xnq_qtensor* qt, size_t m);
 xnq_status xnq_quantize_lhs(uint32_t weight_dtype, size_t m, size_t k, const float* lhs_dev,

@@ -327,7 +327,7 @@ __device__ __forceinline__ void unit_mma(Unit<DT>& u, const h8* a, const Scales<
     u.I = mfma16(a[0], as_h8(b[0]), f16v{});
     u.sc = mfma8(S.d[j], bd);
     u.I = mfma16(a[1], as_h8(b[1]), u.I);
-    if constexpr (HT<DT>::kMin32) u.p = mfma8(S.m[j], chunk_sum(bs, j));
+    if constexpr (HT<DT>::kMin32) u.p = mfma8(S.m[j], bs);
 }
 template <int DT>
 __device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t) {
@@ -342,6 +342,11 @@ __device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t)
         }
     }
 }
+
+// An infinite scale (an infinity in the block) makes every block dot of the
+// reference NaN: a zero sum times it, or main and min terms of one sign.  (The
+// quantizer does the same for the f16 copy.)
+__device__ __forceinline__ float finite_or_nan(float d) { return d - d == 0.0f ? d : d - d; }
 
 // A super-block's sums I (and the min sums) of a 32 x 32 tile into the output.
 template <int DT>
@@ -383,7 +388,33 @@ __device__ __forceinline__ float4 sum_waves(const float4* p, int stride) {
     return make_float4((float)x, (float)y, (float)z, (float)w);
 }
 
-template <int DT, int TM, bool DV>
+// Operand B out of the int8 row images (ActImg) instead of the f16 copy, for callers
+// that hold a quantized activation of their own: the same values, at a conversion
+// beside each product and loads of 16 bytes a row (all of a stage's at once, so
+// that a line is used whole, was no better: Q8_0 4096 -> 1024 m = 125 21 against
+// 20 us, Q5K 4096 -> 6144 m = 37 28 / 21, Q4_0 4096 -> 14336 m = 512 425 / 453).
+__device__ __forceinline__ void row_quants(const uint4& v, uint4* b) {
+    const uint32_t d[4] = {v.x, v.y, v.z, v.w};
+    const h2 c = splat2(-1152.f);  // 1024 + (byte + 128)
+    h2 q[8];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        q[2 * i] = magic01(d[i] ^ 0x80808080u) + c;
+        q[2 * i + 1] = magic23(d[i] ^ 0x80808080u) + c;
+    }
+    b[0] = __builtin_bit_cast(uint4, h8{q[0].x, q[0].y, q[1].x, q[1].y, q[2].x, q[2].y, q[3].x, q[3].y});
+    b[1] = __builtin_bit_cast(uint4, h8{q[4].x, q[4].y, q[5].x, q[5].y, q[6].x, q[6].y, q[7].x, q[7].y});
+}
+__device__ __forceinline__ uint4 row_bsums(const uint4& v) {
+    typedef short s8 __attribute__((ext_vector_type(8)));
+    const s8 t = __builtin_bit_cast(s8, v);
+    h8 h;
+#pragma unroll
+    for (int i = 0; i < 8; i++) h[i] = (_Float16)t[i];  // |bsum| <= 2048: exact
+    return __builtin_bit_cast(uint4, h);
+}
+
+template <int DT, int TM, bool DV, bool ROWS>
 __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, uint32_t m, uint32_t m_tiles,
                                                               uint32_t n_tiles, float* __restrict__ y) {
     using T = HT<DT>;
@@ -411,10 +442,12 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
 
     // lanes of rows past m read the last row again (their outputs are dropped)
     uint32_t rt[TM], bl[TM];
+    const uint8_t* row[TM];  // ROWS: the lane's row image
 #pragma unroll
     for (int i = 0; i < TM; i++) {
-        rt[i] = min(mt * TM + i, H.rts - 1);
+        rt[i] = min(mt * TM + i, ROWS ? (m - 1) / 32 : H.rts - 1);
         bl[i] = g * 32 + min(lrow, m - 1 - rt[i] * 32);
+        if constexpr (ROWS) row[i] = a.img + (size_t)min(rt[i] * 32 + lrow, m - 1) * a.A.row_bytes;
     }
 
     f16v out[TM], mid[TM];
@@ -424,30 +457,65 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
     if (s0 < s1) {
         WOff<DT> wo;
         weight_offsets<DT>(wo, w, col0, lane);
-        uint4 b[kPD][2];
-        uint2 bd[T::kK ? 1 : kPD];
+        uint4 b[kPD][ROWS ? 1 : 2];
+        uint2 bd[T::kK ? 1 : kPD];  // ROWS: f32 scale, quant sum
         float da[TM];    // K types: d_a of the stage's super-block
         uint4 bs[TM];    // and min-term operand
         uint2 bs32[TM];  // Q4_1, Q5_1: min-term operand of the stage
         auto load_unit = [&](uint32_t st, int u, int slot) {
             const int j = u / TM, i = u % TM;
             const uint32_t cj = st * T::kCH + j, c = min(cj, nch - 1);
+            if constexpr (ROWS) {
+                b[slot][0] = *reinterpret_cast<const uint4*>(row[i] + g * (w.k / 2) + c * 16);
+                if constexpr (!T::kK) {  // (no scale past the end of the row)
+                    bd[slot].x = cj < nch ? *reinterpret_cast<const uint32_t*>(row[i] + a.A.d_off + c * 4) : 0u;
+                    if constexpr (T::kMin32) bd[slot].y = *reinterpret_cast<const uint32_t*>(row[i] + a.A.s_off + c * 4);
+                }
+                return;
+            }
             const uint8_t* p = a.h16 + ((size_t)rt[i] * nch + c) * 2048 + bl[i] * 16;
             b[slot][0] = *reinterpret_cast<const uint4*>(p);
-            b[slot][1] = *reinterpret_cast<const uint4*>(p + 1024);
+            if constexpr (!ROWS) b[slot][1] = *reinterpret_cast<const uint4*>(p + 1024);
             if constexpr (!T::kK)
                 bd[slot] = *reinterpret_cast<const uint2*>(a.h16 + H.d_off + ((size_t)rt[i] * nst * 4 + cj) * 512 + lane * 8);
         };
         auto load_scales = [&](uint32_t st) {
 #pragma unroll
             for (int i = 0; i < TM; i++) {
-                if constexpr (T::kK) {
+                if constexpr (ROWS) {
+                    if constexpr (T::kK) {
+                        da[i] = reinterpret_cast<const float*>(row[i] + a.A.d_off)[st];
+                        if constexpr (T::kMinK) bs[i] = *reinterpret_cast<const uint4*>(row[i] + a.A.s_off + st * 32 + g * 16);
+                    }
+                } else if constexpr (T::kK) {
                     da[i] = reinterpret_cast<const float*>(a.h16 + H.d_off + ((size_t)rt[i] * nst + st) * 128)[lrow];
                     if constexpr (T::kMinK)
                         bs[i] = *reinterpret_cast<const uint4*>(a.h16 + H.s_off + ((size_t)rt[i] * nst + st) * 1024 + lane * 16);
                 } else if constexpr (T::kMin32) {
                     bs32[i] = *reinterpret_cast<const uint2*>(a.h16 + H.s_off + ((size_t)rt[i] * nst + st) * 512 + lane * 8);
                 }
+            }
+        };
+        // unit u's operands, as the matrix instructions take them
+        auto unit_b = [&](int u, uint4* ub) {
+            if constexpr (ROWS) {
+                row_quants(b[u % kPD][0], ub);
+            } else {
+                ub[0] = b[u % kPD][0];
+                ub[1] = b[u % kPD][1];
+            }
+        };
+        auto unit_d = [&](int u, uint2& ud, uint2& us) {
+            if constexpr (ROWS) {
+                const float d = __uint_as_float(bd[u % kPD].x);
+                ud = make_uint2(g == 0 ? (uint32_t)f32_to_f16_bits(d) : 0u, 0);
+                if constexpr (T::kMin32) {  // Q8_1's s, as the quantizer forms it
+                    const float t = f16_bits_to_f32(f32_to_f16_bits((float)(int)bd[u % kPD].y));
+                    us = make_uint2(g == 0 ? (uint32_t)f32_to_f16_bits(t * d) : 0u, 0);
+                }
+            } else {
+                ud = bd[u % kPD];
+                if constexpr (T::kMin32) us = chunk_sum(bs32[u % TM], u / TM);
             }
         };
         issue_weights<DT, DV>(wo, w, s0, wbase);
@@ -476,8 +544,10 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
 #pragma unroll
                     for (int i = 0; i < TM; i++) {
                         const int u = j * TM + i;
-                        I[i] = mfma16(A[0], as_h8(b[u % kPD][0]), j == 0 ? f16v{} : I[i]);
-                        I[i] = mfma16(A[1], as_h8(b[u % kPD][1]), I[i]);
+                        uint4 ub[2];
+                        unit_b(u, ub);
+                        I[i] = mfma16(A[0], as_h8(ub[0]), j == 0 ? f16v{} : I[i]);
+                        I[i] = mfma16(A[1], as_h8(ub[1]), I[i]);
                         if (u + kPD < kU) load_unit(s, u + kPD, u % kPD);
                         else load_unit(sn, u + kPD - kU, u % kPD);
                     }
@@ -490,7 +560,12 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
                     if (T::kMinK) dm[e] = dp[32 + 8 * (e >> 2) + (e & 3)];
                 }
 #pragma unroll
-                for (int i = 0; i < TM; i++) super_unit<DT>(I[i], S, bs[i], da[i], dw, dm, out[i]);
+                for (int i = 0; i < TM; i++) {
+                    if constexpr (ROWS)
+                        super_unit<DT>(I[i], S, T::kMinK ? row_bsums(bs[i]) : uint4{}, finite_or_nan(da[i]), dw, dm, out[i]);
+                    else
+                        super_unit<DT>(I[i], S, bs[i], da[i], dw, dm, out[i]);
+                }
             } else {
                 f16v t[TM];
 #pragma unroll
@@ -503,10 +578,16 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
                     for (int i = 0; i < TM; i++) {
                         const int u = j * TM + i;
                         Unit<DT> un;
-                        unit_mma<DT>(un, A, S, j, b[u % kPD], bd[u % kPD], bs32[i]);
+                        uint4 ub[2];
+                        uint2 ud, us{};
+                        unit_b(u, ub);
+                        unit_d(u, ud, us);
+                        unit_mma<DT>(un, A, S, j, ub, ud, us);
                         unit_add<DT>(un, j == 0, t[i]);
                         if (u + kPD < kU) load_unit(s, u + kPD, u % kPD);
                         else load_unit(sn, u + kPD - kU, u % kPD);
+                        // folded here: sunk to the stage's end, with the conversions in front, it spills
+                        if constexpr (ROWS) asm volatile("" : "+v"(t[i]));
                     }
                 }
 #pragma unroll
@@ -1080,7 +1161,7 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             Unit<DT> un;
-            unit_mma<DT>(un, A[j & 1], S, j, b, bd, ms);
+            unit_mma<DT>(un, A[j & 1], S, j, b, bd, T::kMin32 ? chunk_sum(ms, j) : ms);
             __builtin_amdgcn_sched_barrier(0);
             if (j < 3) {
                 read_b(j + 1);
@@ -1122,16 +1203,16 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
     wait_vm<0>();  // no DMA outlives the workgroup's LDS
 }
 
-template <int DT, int TM, bool DV>
+template <int DT, int TM, bool DV, bool ROWS = false>
 hipError_t launch_ksplit(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
     using T = HT<DT>;
     constexpr int kWaveLds = 3 * T::kSlot + T::kDl, kRed = kWaves * TM * 4 * 64 * 16;
     constexpr int kLds = kWaves * kWaveLds > kRed ? kWaves * kWaveLds : kRed;
-    const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_ksplit_kernel<DT, TM, DV>), kLds);
+    const hipError_t e = set_max_lds(reinterpret_cast<const void*>(h16_ksplit_kernel<DT, TM, DV, ROWS>), kLds);
     if (e != hipSuccess) return e;
     const uint32_t n_tiles = (w.n + 31) / 32, rts = (uint32_t)((m + 31) / 32), m_tiles = (rts + TM - 1) / TM;
     const uint32_t grid = (m_tiles * n_tiles + 7) / 8 * 8;
-    h16_ksplit_kernel<DT, TM, DV><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
+    h16_ksplit_kernel<DT, TM, DV, ROWS><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
     return hipGetLastError();
 }
 
@@ -1145,6 +1226,13 @@ hipError_t launch_ksplit16(const WView& w, const AView& a, size_t m, float* y, h
     const uint32_t grid = (m_tiles * n_tiles + 7) / 8 * 8;
     h16_ksplit16_kernel<DT><<<grid, kThreads, kLds, s>>>(w, a, (uint32_t)m, m_tiles, n_tiles, y);
     return hipGetLastError();
+}
+
+template <int DT, bool DV>
+hipError_t launch_rows_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
+    if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV, true>(w, a, m, y, s);
+    return launch_ksplit<DT, 2, DV, true>(w, a, m, y, s);
 }
 
 template <int DT, bool DV>
@@ -1192,20 +1280,34 @@ bool h16_supported(uint32_t dtype) {
     return dtype == XNQ_Q8_0 || dtype == XNQ_Q4_0 || is_raw_layout(dtype);
 }
 
+// launch_h16_dt or launch_rows_dt of the weight's type
+template <bool ROWS>
+static hipError_t launch_type(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+#define XNQ_H16(DT, DV) (ROWS ? launch_rows_dt<DT, DV>(w, a, m, y, s) : launch_h16_dt<DT, DV>(w, a, m, y, s))
+    switch (w.dtype) {
+    case XNQ_Q8_0: return w.nb % 4 == 0 ? XNQ_H16(XNQ_Q8_0, true) : XNQ_H16(XNQ_Q8_0, false);
+    case XNQ_Q4_0: return w.nb % 4 == 0 ? XNQ_H16(XNQ_Q4_0, true) : XNQ_H16(XNQ_Q4_0, false);
+    case XNQ_Q4_1: return XNQ_H16(XNQ_Q4_1, true);
+    case XNQ_Q5_0: return XNQ_H16(XNQ_Q5_0, true);
+    case XNQ_Q5_1: return XNQ_H16(XNQ_Q5_1, true);
+    case XNQ_Q2K: return XNQ_H16(XNQ_Q2K, true);
+    case XNQ_Q3K: return XNQ_H16(XNQ_Q3K, true);
+    case XNQ_Q5K: return XNQ_H16(XNQ_Q5K, true);
+    }
+#undef XNQ_H16
+    return hipErrorNotSupported;
+}
+
 hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (!a.h16 || (size_t)a.H.rts * 32 < m || a.k != w.k) return hipErrorInvalidValue;
-    switch (w.dtype) {
-    case XNQ_Q8_0: return w.nb % 4 == 0 ? launch_h16_dt<XNQ_Q8_0, true>(w, a, m, y, s) : launch_h16_dt<XNQ_Q8_0, false>(w, a, m, y, s);
-    case XNQ_Q4_0: return w.nb % 4 == 0 ? launch_h16_dt<XNQ_Q4_0, true>(w, a, m, y, s) : launch_h16_dt<XNQ_Q4_0, false>(w, a, m, y, s);
-    case XNQ_Q4_1: return launch_h16_dt<XNQ_Q4_1, true>(w, a, m, y, s);
-    case XNQ_Q5_0: return launch_h16_dt<XNQ_Q5_0, true>(w, a, m, y, s);
-    case XNQ_Q5_1: return launch_h16_dt<XNQ_Q5_1, true>(w, a, m, y, s);
-    case XNQ_Q2K: return launch_h16_dt<XNQ_Q2K, true>(w, a, m, y, s);
-    case XNQ_Q3K: return launch_h16_dt<XNQ_Q3K, true>(w, a, m, y, s);
-    case XNQ_Q5K: return launch_h16_dt<XNQ_Q5K, true>(w, a, m, y, s);
-    }
-    return hipErrorNotSupported;
+    return launch_type<false>(w, a, m, y, s);
+}
+
+hipError_t launch_h16_rows(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
+    if (m == 0 || w.n == 0) return hipSuccess;
+    if (a.m < m || a.k != w.k) return hipErrorInvalidValue;
+    return launch_type<true>(w, a, m, y, s);
 }
 
 }  // namespace xnq

@@ -279,9 +279,25 @@ static bool tiled_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
 // to 16 (32-element types) or 32 rows.  m = 8 (f16: 9) and 16, K = 4096, us, matvec / f16:
 // Q8_0 N = 1024 8.0 / 11.3 and 13.2 / 11.3, 14336 22.3 / 26.2 and 41.7 / 26.4; Q4_0
 // 14336 22.8 / 22.3 and 42.7 / 22.4; Q5K 6144 14.1 / 13.7 and 24.5 / 13.8.
-static bool h16_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
-    return forced == 0 && m > 8 && h16_supported(weight_dtype) &&
+static bool h16_rows(uint32_t weight_dtype, size_t m, size_t k) {
+    return m > 8 && h16_supported(weight_dtype) &&
            act_img((uint32_t)k, is_kquant(weight_dtype)).row_bytes <= 160 * 1024;
+}
+static bool h16_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
+    return forced == 0 && h16_rows(weight_dtype, m, k);
+}
+
+// The route of quantize_lhs and matmul_preq.  A caller of the two holds the
+// quantized rows, and may use them with any weight whose type takes the same
+// activation blocks, or use fewer of them: of the f16 kernels' types they are
+// therefore the row images alone, whose layout depends on neither, and
+// matmul_preq (kH16Rows) reads nothing else.  Against the f16 copy that costs a
+// conversion beside each product and 16-byte reads a row, K = 4096, us, graph
+// steps with the quantize, matvec / copy / rows: Q8_0 N = 1024 m = 125 84 / 13 /
+// 20, Q5K 6144 37 55 / 17 / 21, Q4_0 14336 512 1237 / 136 / 453.
+constexpr int kRouteRows = 4;
+static int two_call(uint32_t weight_dtype, int forced) {
+    return forced == 0 && h16_supported(weight_dtype) ? kRouteRows : forced;
 }
 
 ALayout act_layout(uint32_t weight_dtype, size_t m, size_t k, int forced) {
@@ -417,7 +433,7 @@ size_t xnq_qtensor_device_bytes(const xnq_qtensor* qt) { return qt ? qt->L.bytes
 
 size_t xnq_lhs_workspace_size(uint32_t weight_dtype, size_t m, size_t k) {
     if (!device_dtype(weight_dtype)) return 0;
-    return act_layout(weight_dtype, m, k, g_route.load()).bytes;
+    return act_layout(weight_dtype, m, k, two_call(weight_dtype, g_route.load())).bytes;
 }
 
 static xnq_status check_lhs(uint32_t weight_dtype, size_t k) {
@@ -445,7 +461,7 @@ static xnq_status quantize_lhs_impl(uint32_t weight_dtype, size_t m, size_t k, c
 
 xnq_status xnq_quantize_lhs(uint32_t weight_dtype, size_t m, size_t k, const float* lhs_dev,
                             void* workspace_dev, void* stream) {
-    return quantize_lhs_impl(weight_dtype, m, k, lhs_dev, workspace_dev, stream, g_route.load());
+    return quantize_lhs_impl(weight_dtype, m, k, lhs_dev, workspace_dev, stream, two_call(weight_dtype, g_route.load()));
 }
 
 xnq_status xnq_set_route(int route) {
@@ -482,7 +498,7 @@ static xnq_status check_mkn(const xnq_qtensor* qt, size_t m, size_t k, size_t n)
 // tuning (read once per process); `forced` is xnq_set_route's override as
 // read at the entry point; `group_n` is the joined width of a group (0 for a
 // single weight).
-enum Route { kMatvec, kSkinny, kMfma, kH16 };
+enum Route { kMatvec, kSkinny, kMfma, kH16, kH16Rows };
 
 static Route pick_route(uint32_t dtype, size_t m, size_t n, size_t k, int forced, size_t group_n = 0) {
     static const size_t skinny_min = env_size("XNQ_SKINNY_MIN_ROWS", 0);
@@ -491,6 +507,7 @@ static Route pick_route(uint32_t dtype, size_t m, size_t n, size_t k, int forced
     if (forced == 2) return kMfma;
     if (forced == 3) return kSkinny;
     if (h16_act(dtype, m, k, forced)) return kH16;
+    if (forced == kRouteRows && h16_rows(dtype, m, k)) return kH16Rows;
     // measured crossovers (graph steps, µs, matvec against skinny): the
     // matvec kernels' cost jumps from 4 to 5 rows (the 8-row template) and
     // past 8 rows takes a second launch; the skinny kernel's hardly grows
@@ -539,7 +556,7 @@ static size_t workspace_size_impl(const xnq_qtensor* qt, size_t m, int forced) {
 }
 
 size_t xnq_qtensor_workspace_size(const xnq_qtensor* qt, size_t m) {
-    return workspace_size_impl(qt, m, g_route.load());
+    return qt ? workspace_size_impl(qt, m, two_call(qt->L.dtype, g_route.load())) : 0;
 }
 
 static xnq_status matmul_preq_impl(const xnq_qtensor* qt, size_t m, size_t k, size_t n, const void* workspace_dev,
@@ -565,6 +582,8 @@ static xnq_status matmul_preq_impl(const xnq_qtensor* qt, size_t m, size_t k, si
                        : launch_skinny(w, a, m, splits, dst_dev, partial, (hipStream_t)stream);
     } else if (r == kH16) {
         e = launch_h16(w, a, m, dst_dev, (hipStream_t)stream);
+    } else if (r == kH16Rows) {
+        e = launch_h16_rows(w, a, m, dst_dev, (hipStream_t)stream);
     } else {
         e = launch_matvec(w, a, m, dst_dev, (hipStream_t)stream);
     }
@@ -577,7 +596,9 @@ static xnq_status matmul_preq_impl(const xnq_qtensor* qt, size_t m, size_t k, si
 xnq_status xnq_qtensor_matmul_preq(const xnq_qtensor* qt, size_t m, size_t k, size_t n,
                                    const void* workspace_dev, size_t workspace_bytes, float* dst_dev,
                                    void* stream) {
-    return matmul_preq_impl(qt, m, k, n, workspace_dev, workspace_bytes, dst_dev, stream, g_route.load());
+    const int route = g_route.load();
+    return matmul_preq_impl(qt, m, k, n, workspace_dev, workspace_bytes, dst_dev, stream,
+                            qt ? two_call(qt->L.dtype, route) : route);
 }
 
 // Decode: the fused matvec route quantizes the activation row in LDS inside
@@ -1101,7 +1122,7 @@ xnq_status xnq_qtensor_block_ints(const xnq_qtensor* qt, size_t m, const void* w
     if (!workspace_dev || !out_dev) return fail(XNQ_ERR_INVALID, "null pointer");
     DeviceGuard g(qt->device);
     const WView w = make_wview(qt->L, qt->buf);
-    const AView a = make_aview(act_layout(qt->L.dtype, m, qt->L.k, g_route.load()), workspace_dev);
+    const AView a = make_aview(act_layout(qt->L.dtype, m, qt->L.k, two_call(qt->L.dtype, g_route.load())), workspace_dev);
     hipError_t e = launch_block_ints(w, a, m, out_dev, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "block_ints");
     return XNQ_OK;

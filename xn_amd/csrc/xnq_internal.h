@@ -321,5 +321,7 @@ hipError_t launch_prefill(const WView& w, const AView& a, size_t m, uint32_t spl
 // k_h16.hip: the f16 matrix-core kernels of the other weight types
 bool h16_supported(uint32_t dtype);
 hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s);
+// the same from the row images alone
+hipError_t launch_h16_rows(const WView& w, const AView& a, size_t m, float* y, hipStream_t s);
 
 }  // namespace xnq
