@@ -81,3 +81,36 @@ def test_nonfinite_rows(orc, dev, dt, k, m, n):
     ok = want.isfinite().all(1)
     assert ok.sum() >= m - 5 and (got[13] == 0).all()
     assert ((got[ok] - want[ok]).double().norm() / want[ok].double().norm()).item() < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [Q4_1, Q8_0, Q2K, Q5K])
+def test_workspace_of_the_row_images(orc, dev, dt):
+    """matmul_t_ws and a group take a workspace of the row images' size (what
+    workspace() gives), and refuse a smaller one."""
+    import ctypes
+
+    from xn_amd import GgmlDType, QTensor, XnqError, _lib
+    from xn_amd._lib import check
+
+    m, k, n = 40, 512, 96
+    rng = np.random.default_rng(930 + dt)
+    blocks = [orc.from_float(dt, rng.normal(0, 0.02, (n, k)).astype(np.float32)) for _ in range(2)]
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    qts = [QTensor.from_gguf_bytes(b, (n, k), GgmlDType(dt), dev) for b in blocks]
+    want = [orc.matmul(dt, x, b, n).astype(np.float64) for b in blocks]
+    xt, ys, ws = torch.from_numpy(x).to(dev), [torch.full((m, n), float("nan"), device=dev) for _ in qts], qts[0].workspace(m)
+    assert ws.numel() < qts[0].matmul_t_workspace_size(m)
+
+    def close(y, w):
+        return np.linalg.norm(y.cpu().numpy().astype(np.float64) - w) < 2e-6 * np.linalg.norm(w)
+
+    qts[0].matmul_t_ws((m, k, n), xt, ws, ys[0])
+    assert close(ys[0], want[0])
+    with pytest.raises(XnqError, match="smaller"):
+        qts[0].matmul_t_ws((m, k, n), xt, ws[:-256], ys[0])
+    hs = (ctypes.c_void_p * 2)(*[q.storage.handle.value for q in qts])
+    ds = (ctypes.c_void_p * 2)(*[y.fill_(float("nan")).data_ptr() for y in ys])
+    check(_lib.load().xnq_matmul_t_group(hs, 2, m, k, xt.data_ptr(), ds, ws.data_ptr(), ws.numel(),
+                                         torch.cuda.current_stream().cuda_stream))
+    assert close(ys[0], want[0]) and close(ys[1], want[1])

@@ -666,7 +666,13 @@ static xnq_status matmul_t_ws_impl(const xnq_qtensor* qt, size_t m, size_t k, si
         if (e != hipSuccess) return hip_fail(e, "matvec kernel");
         return XNQ_OK;
     }
-    const size_t need = act_layout(qt->L.dtype, m, k, forced).bytes;
+    size_t need = act_layout(qt->L.dtype, m, k, forced).bytes;
+    if (workspace_bytes < need) {
+        // one that holds the row images but not the f16 copy of the rows (all that
+        // these types took with the matvec kernels) serves as in matmul_preq
+        forced = two_call(qt->L.dtype, forced);
+        need = act_layout(qt->L.dtype, m, k, forced).bytes;
+    }
     if (!workspace_dev || workspace_bytes < need)
         return fail(XNQ_ERR_INVALID, "workspace of %zu bytes is smaller than the %zu the activation needs",
                     workspace_bytes, need);
@@ -1046,16 +1052,21 @@ xnq_status xnq_matmul_t_group(const xnq_qtensor* const* qts, size_t count, size_
                                 forced);
     if (shared_quantize(qts, count, m, forced)) {
         // one activation image for every weight, then one matmul each
-        const size_t need = act_layout(qts[0]->L.dtype, m, k, forced).bytes;
+        int route = forced;
+        size_t need = act_layout(qts[0]->L.dtype, m, k, route).bytes;
+        if (workspace_bytes < need) {  // as in matmul_t_ws
+            route = two_call(qts[0]->L.dtype, forced);
+            need = act_layout(qts[0]->L.dtype, m, k, route).bytes;
+        }
         if (!workspace_dev || workspace_bytes < need)
             return fail(XNQ_ERR_INVALID, "workspace of %zu bytes is smaller than the %zu the activation needs",
                         workspace_bytes, need);
         DeviceGuard g(qts[0]->device);
         if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
-        xnq_status st = quantize_lhs_impl(qts[0]->L.dtype, m, k, lhs_dev, workspace_dev, stream, forced);
+        xnq_status st = quantize_lhs_impl(qts[0]->L.dtype, m, k, lhs_dev, workspace_dev, stream, route);
         for (size_t i = 0; i < count && !st; i++)
             st = matmul_preq_impl(qts[i], m, k, qts[i]->L.n, workspace_dev, workspace_bytes, dsts_dev[i], stream,
-                                  forced);
+                                  route);
         return st;
     }
     for (size_t i = 0; i < count; i++) {
