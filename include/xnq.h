@@ -134,9 +134,10 @@ xnq_status xnq_qtensor_matmul_t_ws(const xnq_qtensor* qt, size_t m, size_t k, si
  * XNQ_NOALLOC_SCRATCH_BYTES per GPU that the library holds until the
  * process ends.  Fails with XNQ_ERR_INVALID when
  * xnq_qtensor_matmul_t_workspace_size(qt, m) exceeds it (at K = 4096 that
- * is past about 3000 rows of Q4_K), not counting the f16 copy of the rows
- * that the f16 MFMA kernels read: such a call runs in slabs of rows (Q8_0
- * at K = 4096 up to about 13000 rows, as one launch up to about 4300).
+ * is past about 3000 rows of Q4_K), not counting what the rows take as
+ * f16 (for the f16 MFMA kernels) beyond their 8-bit images: such a call runs
+ * in slabs of rows (Q8_0 at K = 4096 up to about 13000 rows, as one launch up
+ * to about 6500).
  * Every call on one GPU uses that GPU's one array: calls that overlap on one
  * GPU (different streams, or host threads without ordering between them)
  * race and must be serialised by the caller, e.g. by issuing them on one

@@ -345,7 +345,7 @@ __device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t)
 
 // An infinite scale (an infinity in the block) makes every block dot of the
 // reference NaN: a zero sum times it, or main and min terms of one sign.  (The
-// quantizer does the same for the f16 copy.)
+// quantizer does the same for the f16 image.)
 __device__ __forceinline__ float finite_or_nan(float d) { return d - d == 0.0f ? d : d - d; }
 
 // A super-block's sums I (and the min sums) of a 32 x 32 tile into the output.
@@ -388,7 +388,7 @@ __device__ __forceinline__ float4 sum_waves(const float4* p, int stride) {
     return make_float4((float)x, (float)y, (float)z, (float)w);
 }
 
-// Operand B out of the int8 row images (ActImg) instead of the f16 copy, for callers
+// Operand B out of the int8 row images (ActImg) instead of the f16 image, for callers
 // that hold a quantized activation of their own: the same values, at a conversion
 // beside each product and loads of 16 bytes a row (all of a stage's at once, so
 // that a line is used whole, was no better: Q8_0 4096 -> 1024 m = 125 21 against

@@ -126,10 +126,9 @@ __global__ __launch_bounds__(256) void quantize_q80_kernel(const float* __restri
 }
 
 // ---------------------------------------------------------------------------
-// Activations for the f16 matrix-core kernels: the row image plus its f16 copy
-// in MFMA operand order (H16Img).  A workgroup takes 8 rows, so that every
-// (chunk, step, half) piece it assembles in LDS is one whole 128-byte line of
-// the copy.  Rows past m (the padding of the last 32-row tile) are zeros.
+// Activations for the f16 matrix-core kernels: the quantized rows as f16 in MFMA
+// operand order (H16Img).  A workgroup takes 8 rows, so that every (chunk, step,
+// half) piece it assembles in LDS is one whole 128-byte line of the image.  Rows past m (the padding of the last 32-row tile) are zeros.
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ uint2 quants_f16(uint32_t packed) {
     typedef _Float16 v4h_t __attribute__((ext_vector_type(4)));
@@ -139,17 +138,15 @@ __device__ __forceinline__ uint2 quants_f16(uint32_t packed) {
     return __builtin_bit_cast(uint2, h);
 }
 
-__global__ __launch_bounds__(512) void quantize_q8k_h16_kernel(const float* __restrict__ x, uint32_t m, ActImg A,
-                                                               uint8_t* __restrict__ out, uint8_t* __restrict__ img,
-                                                               H16Img H) {
+__global__ __launch_bounds__(512) void quantize_q8k_h16_kernel(const float* __restrict__ x, uint32_t m, uint32_t k,
+                                                               uint8_t* __restrict__ img, H16Img H) {
     __shared__ __align__(16) uint8_t sq[32 * 128];  // [chunk 8][step 2][half 2][row 8][16]
     __shared__ __align__(16) _Float16 ss[2][8][8];  // bsums [half][row][8]
     const int lane = threadIdx.x & (kWave - 1), rr = threadIdx.x / kWave;
-    const uint32_t nsb = A.k / 256, sb = blockIdx.x % nsb, grp = blockIdx.x / nsb, row = grp * 8 + rr;
-    const float4 v = row < m ? reinterpret_cast<const float4*>(x + (size_t)row * A.k + (size_t)sb * 256)[lane]
+    const uint32_t nsb = k / 256, sb = blockIdx.x % nsb, grp = blockIdx.x / nsb, row = grp * 8 + rr;
+    const float4 v = row < m ? reinterpret_cast<const float4*>(x + (size_t)row * k + (size_t)sb * 256)[lane]
                              : make_float4(0.f, 0.f, 0.f, 0.f);
     const Q8KLane r = q8k_quant_wave(v, lane);
-    if (row < m) q8k_store(out + (size_t)row * A.row_bytes, A, sb, lane, r);
     const int sub = lane & 7, piece = (((lane >> 3) * 2 + ((sub >> 1) & 1)) * 2) + (sub >> 2);
     *reinterpret_cast<uint2*>(sq + piece * 128 + rr * 16 + (sub & 1) * 8) = quants_f16(r.packed);
     const size_t rt = grp / 4, r32 = (grp & 3) * 8;
@@ -173,18 +170,16 @@ __global__ __launch_bounds__(512) void quantize_q8k_h16_kernel(const float* __re
 
 // Q8_0 / Q8_1 blocks: one wavefront per (8 rows, chunk), four chunks (a stage)
 // per workgroup.  `mins`: also Q8_1's s (f16 of f16(sum) * d, k_quants.rs:871).
-__global__ __launch_bounds__(256) void quantize_q80_h16_kernel(const float* __restrict__ x, uint32_t m, ActImg A,
-                                                               uint8_t* __restrict__ out, uint8_t* __restrict__ img,
-                                                               H16Img H, int mins) {
+__global__ __launch_bounds__(256) void quantize_q80_h16_kernel(const float* __restrict__ x, uint32_t m, uint32_t k,
+                                                               uint8_t* __restrict__ img, H16Img H, int mins) {
     __shared__ __align__(16) uint8_t sq[4][4 * 128];  // [chunk][step 2][half 2][row 8][16]
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave, rr = lane >> 3, sub = lane & 7;
-    const uint32_t nch = A.k / 32, nst = (nch + 3) / 4, st = blockIdx.x % nst, grp = blockIdx.x / nst;
+    const uint32_t nch = k / 32, nst = (nch + 3) / 4, st = blockIdx.x % nst, grp = blockIdx.x / nst;
     const uint32_t row = grp * 8 + rr, c = st * 4 + wave;
     const bool live = c < nch;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (live && row < m) v = reinterpret_cast<const float4*>(x + (size_t)row * A.k + (size_t)c * 32)[sub];
+    if (live && row < m) v = reinterpret_cast<const float4*>(x + (size_t)row * k + (size_t)c * 32)[sub];
     const Q80Lane r = q80_quant_8lanes(v);
-    if (live && row < m) q80_store(out + (size_t)row * A.row_bytes, A, c, sub, r);
     *reinterpret_cast<uint2*>(sq[wave] + (((sub >> 1) & 1) * 2 + (sub >> 2)) * 128 + rr * 16 + (sub & 1) * 8) =
         quants_f16(r.packed);
     const size_t rt = grp / 4, r32 = (grp & 3) * 8 + rr;
@@ -808,13 +803,12 @@ hipError_t launch_quantize_act(const ALayout& L, const float* x, void* ws, hipSt
     uint8_t* b = static_cast<uint8_t*>(ws);
     if (L.m == 0) return hipSuccess;
     if (L.h16) {
-        uint8_t* img = b + L.h16_off;
         if (L.act_dtype == XNQ_Q8K)
-            quantize_q8k_h16_kernel<<<(unsigned)(L.himg.rts * 4 * (L.k / 256)), 512, 0, s>>>(x, (uint32_t)L.m, L.img, b,
-                                                                                            img, L.himg);
+            quantize_q8k_h16_kernel<<<(unsigned)(L.himg.rts * 4 * (L.k / 256)), 512, 0, s>>>(x, (uint32_t)L.m,
+                                                                                            (uint32_t)L.k, b, L.himg);
         else
             quantize_q80_h16_kernel<<<(unsigned)(L.himg.rts * 4 * ((L.k / 32 + 3) / 4)), 256, 0, s>>>(
-                x, (uint32_t)L.m, L.img, b, img, L.himg, L.act_dtype == XNQ_Q8_1);
+                x, (uint32_t)L.m, (uint32_t)L.k, b, L.himg, L.act_dtype == XNQ_Q8_1);
     } else if (L.act_dtype == XNQ_Q8K) {
         const size_t nblocks = L.m * (L.k / 256);
         if (L.tiled)

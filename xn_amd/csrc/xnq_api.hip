@@ -272,7 +272,7 @@ static bool tiled_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
 }
 
 // Whether m rows take the f16 matrix-core kernels (the activation quantizer
-// then also writes the f16 copy of the rows); like tiled_act a function of the
+// then writes the rows as f16 only); like tiled_act a function of the
 // type, m and K only.  K is bounded as for the matvec kernels, whose LDS holds
 // a row image.  The matvec kernels take up to 8 rows in one launch and read
 // the weights again for every further 8; the f16 kernels cost the same from 1
@@ -291,9 +291,9 @@ static bool h16_act(uint32_t weight_dtype, size_t m, size_t k, int forced) {
 // quantized rows, and may use them with any weight whose type takes the same
 // activation blocks, or use fewer of them: of the f16 kernels' types they are
 // therefore the row images alone, whose layout depends on neither, and
-// matmul_preq (kH16Rows) reads nothing else.  Against the f16 copy that costs a
+// matmul_preq (kH16Rows) reads nothing else.  Against the f16 image that costs a
 // conversion beside each product and 16-byte reads a row, K = 4096, us, graph
-// steps with the quantize, matvec / copy / rows: Q8_0 N = 1024 m = 125 84 / 13 /
+// steps with the quantize, matvec / f16 image / rows: Q8_0 N = 1024 m = 125 84 / 13 /
 // 20, Q5K 6144 37 55 / 17 / 21, Q4_0 14336 512 1237 / 136 / 453.
 constexpr int kRouteRows = 4;
 static int two_call(uint32_t weight_dtype, int forced) {
@@ -315,9 +315,8 @@ ALayout act_layout(uint32_t weight_dtype, size_t m, size_t k, int forced) {
     }
     if (h16_act(weight_dtype, m, k, forced)) {
         L.h16 = true;
-        L.h16_off = L.bytes;
         L.himg = h16_img(m, (uint32_t)k, L.act_dtype == XNQ_Q8K, L.act_dtype == XNQ_Q8_1);
-        L.bytes = align_up(L.h16_off + L.himg.bytes);
+        L.bytes = align_up(L.himg.bytes);
     }
     return L;
 }
@@ -668,8 +667,8 @@ static xnq_status matmul_t_ws_impl(const xnq_qtensor* qt, size_t m, size_t k, si
     }
     size_t need = act_layout(qt->L.dtype, m, k, forced).bytes;
     if (workspace_bytes < need) {
-        // one that holds the row images but not the f16 copy of the rows (all that
-        // these types took with the matvec kernels) serves as in matmul_preq
+        // one that holds the row images but not the f16 image (all that these types
+        // took with the matvec kernels) serves as in matmul_preq
         forced = two_call(qt->L.dtype, forced);
         need = act_layout(qt->L.dtype, m, k, forced).bytes;
     }
@@ -746,8 +745,8 @@ xnq_status xnq_qtensor_matmul_t_noalloc(const xnq_qtensor* qt, size_t m, size_t 
     if (st) return st;
     const int forced = g_route.load();
     const size_t need = matmul_t_workspace_size_impl(qt, m, forced);
-    // The f16 route's copy of the rows fills the scratch from fewer rows on than
-    // the row images alone: up to the rows whose images fit, it runs in slabs
+    // The f16 image of the rows fills the scratch from fewer rows on than the
+    // row images did: up to the rows whose images fit, it runs in slabs
     // (the rows are independent).
     const bool slabs = need > XNQ_NOALLOC_SCRATCH_BYTES && pick_route(qt->L.dtype, m, n, k, forced) == kH16 &&
                        act_layout(qt->L.dtype, m, k, 1).bytes <= XNQ_NOALLOC_SCRATCH_BYTES;

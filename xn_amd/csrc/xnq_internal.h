@@ -147,7 +147,7 @@ __host__ __device__ inline TileImg tile_img(size_t m, uint32_t k) {
     return T;
 }
 
-// f16 copy of the quantized rows for the f16 matrix-core kernels (k_h16.hip),
+// The quantized rows as f16 for the f16 matrix-core kernels (k_h16.hip),
 // in MFMA operand order: rows in tiles of 32 (the last one padded with zero
 // rows), lane = 32 * half + row, every piece one contiguous KiB (or less):
 //   quants  [tile][chunk c][step 2][lane 64][16]: elements 16 half + 8 step ..
@@ -182,8 +182,7 @@ struct ALayout {
     bool tiled = false;  // a TileImg follows the row images at tile_off
     size_t tile_off = 0;
     TileImg tile{};
-    bool h16 = false;  // an H16Img follows the row images at h16_off
-    size_t h16_off = 0;
+    bool h16 = false;  // an H16Img in the place of the row images
     H16Img himg{};
 };
 
@@ -193,7 +192,7 @@ struct AView {
     ActImg A;
     const uint8_t* tile;  // null unless the layout is tiled
     TileImg T;
-    const uint8_t* h16;  // null unless the layout has the f16 copy
+    const uint8_t* h16;  // null unless the layout is the f16 one (then there are no row images)
     H16Img H;
 };
 
@@ -238,13 +237,13 @@ inline WView make_wview(const WLayout& L, const void* base) {
 
 inline AView make_aview(const ALayout& L, const void* base) {
     AView v;
-    v.img = static_cast<const uint8_t*>(base);
+    v.img = L.h16 ? nullptr : static_cast<const uint8_t*>(base);
     v.m = (uint32_t)L.m;
     v.k = (uint32_t)L.k;
     v.A = L.img;
     v.tile = L.tiled ? v.img + L.tile_off : nullptr;
     v.T = L.tile;
-    v.h16 = L.h16 ? v.img + L.h16_off : nullptr;
+    v.h16 = L.h16 ? static_cast<const uint8_t*>(base) : nullptr;
     v.H = L.himg;
     return v;
 }
