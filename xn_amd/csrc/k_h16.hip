@@ -3,12 +3,12 @@
 // from a few rows up to prefill sizes.
 //
 // Exactness.  Every level of these formats times its integer sub-block scale
-// (Q5K: 6-bit scale x 5-bit level <= 1953) and every 8-bit activation level
-// is a whole number that f16 holds exactly, their products are exact, and
-// the sum of one block (|I| < 2^24) is exact in the f32 accumulator: the
-// matrix core returns the same integer block dot the reference forms
-// (k_quants.rs:287-304, 419-440, 513-544, 677-691, 899-948, 1071-1152,
-// 1524-1605), as a float and without a conversion.
+// and every 8-bit activation level is a whole number that f16 holds exactly,
+// and their products are exact.  The sum of one block is below 2^24 (Q8_0
+// 5.2e5, Q2K 1.5e6, Q3K 4.2e6) and so exact in the f32 accumulator: the matrix
+// core returns the same integer block dot the reference forms (k_quants.rs:
+// 287-304, 419-440, 513-544, 677-691, 899-948, 1071-1152, 1524-1605), as a float
+// and without a conversion.  Q5K's can reach 63 x 31 x 128 x 256 = 6.4e7, see there.
 //
 // Scales.  The 32-element types scale every 32 K: y += (d_w d_a) I.  Both
 // scales are f16, so their outer product over a 32 x 32 tile is one more
@@ -17,6 +17,16 @@
 // two, and with an int8 contraction three).  The K types scale every 256 K:
 // y += d_a (d_w I1 - dmin I2), where I2 = sum_g m_g bsum_g is one K = 16 MFMA
 // of the sub-block mins by the 16 block sums, exact for the same reason.
+//
+// Q5K.  On activations of one sign I1 passes 2^24, and d_w I1 and dmin I2 are
+// several times their difference.  The levels are therefore expanded less 16,
+// which keeps the running sum small, and one more MFMA adds
+// sum_g (16 sc_g - kappa m_g) bsum_g with kappa = dmin / d_w rounded to a whole number
+// of 0 .. 31, so that the larger part of the cancellation is between whole numbers
+// (below 2^24 unless a whole block's levels are extreme); what the min term then
+// still has is dmin - kappa d_w.  Relative L2 error against 64 bits on rows of 10 + 0.3 N(0, 1),
+// matvec / with levels 0 .. 31 / this: K = 256 1.48e-7 / 2.62e-7 / 3.8e-8, 4096
+// 1.60e-7 / 2.73e-7 / 4.7e-8; on N(0, 1) rows 4096 1.04e-7 / 6.2e-8 / 4.8e-8.
 //
 // Operands.  Weight columns are MFMA operand A (expanded to f16 in registers
 // right before use: a nibble or byte b becomes 0x6400 | b = 1024 + b, then one
@@ -82,6 +92,13 @@ __device__ __forceinline__ h2 magic01(uint32_t x) {
 }
 __device__ __forceinline__ h2 magic23(uint32_t x) {
     return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, x, 0x04030402u));
+}
+// 256 + byte / 4 for bytes (0, 1) and (2, 3) of x
+__device__ __forceinline__ h2 quarter01(uint32_t x) {
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x5c5c5c5cu, x, 0x04010400u));
+}
+__device__ __forceinline__ h2 quarter23(uint32_t x) {
+    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x5c5c5c5cu, x, 0x04030402u));
 }
 __device__ __forceinline__ h2 splat2(float v) {
     const _Float16 h = (_Float16)v;
@@ -166,10 +183,22 @@ __device__ __forceinline__ void read_chunk(Bytes& r, const uint8_t* slot, uint32
     }
 }
 
-// Operand A of chunk j: the lane's 16 levels (times the sub-block scale, K
-// types) as two K = 16 steps; hd the block header words a K type needs.
+// What a stage needs of its weights beside the levels.
 template <int DT>
-__device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const uint4& hd, h8* a) {
+struct Scales {
+    uint4 hd;                            // K types: the block header's words
+    uint2 d[HT<DT>::kK ? 1 : 4];      // 32-element types: operand of the scale product, chunk j
+    uint2 m[HT<DT>::kMin32 ? 4 : 1];  // and of the min product
+    uint4 mn;                            // K types: min-term operand
+    uint4 rest;                          // Q5K: 16 sc - kappa m, laid out like it,
+    float bias;                          // and -272, or -256 where d_w is not finite
+};
+
+// Operand A of chunk j: the lane's 16 levels (times the sub-block scale, K
+// types) as two K = 16 steps.
+template <int DT>
+__device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const Scales<DT>& S, h8* a) {
+    const uint4& hd = S.hd;
     const uint32_t v[4] = {r.v.x, r.v.y, r.v.z, r.v.w}, w[4] = {r.w.x, r.w.y, r.w.z, r.w.w};
     uint32_t x[4];  // four levels a dword, as bytes
     float bias = 0.f, sc = 0.f;
@@ -186,8 +215,8 @@ __device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const 
         bias = DT == XNQ_Q4_0 ? -1032.f : DT == XNQ_Q5_0 ? -1040.f : -1024.f;
     } else if constexpr (DT == XNQ_Q5K) {
 #pragma unroll
-        for (int d = 0; d < 4; d++)
-            x[d] = ((v[d] >> (4 * (j & 1))) & 0x0F0F0F0Fu) | ((j >= 4 ? w[d] >> (j - 4) : w[d] << (4 - j)) & 0x10101010u);
+        for (int d = 0; d < 4; d++)  // four times the level
+            x[d] = ((j & 1 ? v[d] >> 2 : v[d] << 2) & 0x3C3C3C3Cu) | ((j > 6 ? w[d] >> 1 : w[d] << (6 - j)) & 0x40404040u);
         const Q4KScales q = q4k_scales(hd.y, hd.z, hd.w);
         sc = (float)(((j < 4 ? q.sc_lo : q.sc_hi) >> (8 * (j & 3))) & 0xffu);
     } else {
@@ -205,8 +234,8 @@ __device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const 
     h2 q[8];
 #pragma unroll
     for (int d = 0; d < 4; d++) {
-        q[2 * d] = magic01(x[d]);
-        q[2 * d + 1] = magic23(x[d]);
+        q[2 * d] = DT == XNQ_Q5K ? quarter01(x[d]) : magic01(x[d]);
+        q[2 * d + 1] = DT == XNQ_Q5K ? quarter23(x[d]) : magic23(x[d]);
     }
     if constexpr (!HT<DT>::kK) {
         const h2 b = splat2(bias);
@@ -217,8 +246,9 @@ __device__ __forceinline__ void expand(const Bytes& r, int j, uint32_t h, const 
 #pragma unroll
         for (int d = 0; d < 8; d++) q[d] = (q[d] + b) * s;
     } else {
-        // (1024 + q) sc - 1024 sc, exact: 1024 sc is a 6-bit number times 2^10
-        const h2 s = splat2(sc), b = splat2(-1024.f * sc);
+        // Q2K (1024 + q) sc - 1024 sc, Q5K (256 + q) sc - 272 sc = (q - 16) sc, exact: 1024 sc
+        // is a 4-bit number times 2^10, 272 sc = 17 sc <= 1071 times 2^4
+        const h2 s = splat2(sc), b = splat2((DT == XNQ_Q5K ? S.bias : -1024.f) * sc);
 #pragma unroll
         for (int d = 0; d < 8; d++) q[d] = __builtin_elementwise_fma(q[d], s, b);
     }
@@ -234,15 +264,6 @@ __device__ __forceinline__ f16v mfma8(uint2 a, uint2 b) {
     return __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(h4, a), __builtin_bit_cast(h4, b), f16v{}, 0, 0, 0);
 }
 __device__ __forceinline__ h8 as_h8(uint4 v) { return __builtin_bit_cast(h8, v); }
-
-// What a stage needs of its weights beside the levels.
-template <int DT>
-struct Scales {
-    uint4 hd;                            // K types: the block header's words
-    uint2 d[HT<DT>::kK ? 1 : 4];      // 32-element types: operand of the scale product, chunk j
-    uint2 m[HT<DT>::kMin32 ? 4 : 1];  // and of the min product
-    uint4 mn;                            // K types: min-term operand
-};
 
 // Reads a stage's scales from its slot; K types also leave d_w and dmin by
 // column at dl (a wavefront's own LDS: its operations stay in order).
@@ -264,20 +285,18 @@ __device__ __forceinline__ void read_scales(Scales<DT>& S, const WView& w, const
             S.hd = lds16(col + 96);
             dd = S.hd.w & 0xffffu;
         }
-        reinterpret_cast<float*>(dl)[lane] = f16_bits_to_f32(h ? dd >> 16 : dd & 0xffffu);  // [dw 32][dmin 32]
-        if constexpr (T::kMinK) {
+        if constexpr (DT == XNQ_Q5K) {  // (the rest: read_rest)
+            const float dw = f16_bits_to_f32(dd & 0xffffu);
+            S.bias = dw - dw == 0.f ? -272.f : -256.f;
+        } else {
+            reinterpret_cast<float*>(dl)[lane] = f16_bits_to_f32(h ? dd >> 16 : dd & 0xffffu);  // [dw 32][dmin 32]
+        }
+        if constexpr (DT == XNQ_Q2K) {
             // mins of sub-blocks (16 elements each) 8h .. 8h + 7
             h8 mv;
-            if constexpr (DT == XNQ_Q5K) {
-                const Q4KScales q = q4k_scales(S.hd.y, S.hd.z, S.hd.w);
-                const uint32_t mw = h ? q.m_hi : q.m_lo;
+            const uint32_t b0 = h ? S.hd.z : S.hd.x, b1 = h ? S.hd.w : S.hd.y;
 #pragma unroll
-                for (int t = 0; t < 8; t++) mv[t] = (_Float16)(float)((mw >> (8 * (t >> 1))) & 0xffu);
-            } else {
-                const uint32_t b0 = h ? S.hd.z : S.hd.x, b1 = h ? S.hd.w : S.hd.y;
-#pragma unroll
-                for (int t = 0; t < 8; t++) mv[t] = (_Float16)(float)(((t < 4 ? b0 : b1) >> (8 * (t & 3) + 4)) & 15u);
-            }
+            for (int t = 0; t < 8; t++) mv[t] = (_Float16)(float)(((t < 4 ? b0 : b1) >> (8 * (t & 3) + 4)) & 15u);
             S.mn = __builtin_bit_cast(uint4, mv);
         }
     } else {
@@ -343,6 +362,36 @@ __device__ __forceinline__ void unit_add(const Unit<DT>& u, bool first, f16v& t)
     }
 }
 
+// Each byte of w (<= 63) times f (1 or 16) as two f16 whole numbers.
+__device__ __forceinline__ void bytes_twice(uint32_t w, float f, h2* r) {
+#pragma unroll
+    for (int t = 0; t < 4; t++) {  // (1024 + byte) f - 1024 f
+        const h2 v = __builtin_bit_cast(h2, __builtin_amdgcn_perm(0x64646464u, w, 0x04000400u + 0x00010001u * t));
+        r[t] = __builtin_elementwise_fma(v, splat2(f), splat2(-1024.f * f));
+    }
+}
+
+// Q5K: the operands of the block sums, and at dl d_w and what kappa d_w leaves of dmin.
+// Apart from read_scales: nothing needs them before the super-block's products are done.
+template <int DT>
+__device__ __forceinline__ void read_rest(Scales<DT>& S, uint8_t* dl, uint32_t lane) {
+    const uint32_t h = lane >> 5;
+    const Q4KScales q = q4k_scales(S.hd.y, S.hd.z, S.hd.w);
+    const float dw = f16_bits_to_f32(S.hd.x & 0xffffu), dm = f16_bits_to_f32(S.hd.x >> 16);
+    const bool ok = dw - dw == 0.f;
+    // (any whole number would be right: an infinite or NaN quotient is clamped, d_w's own
+    // infinity or NaN meets the sums as they are)
+    const float kappa = ok ? rintf(fminf(fmaxf(dm * __builtin_amdgcn_rcpf(dw), 0.f), 31.f)) : 0.f;
+    h2 m[4], c[4];
+    bytes_twice(h ? q.m_hi : q.m_lo, 1.f, m);
+    bytes_twice(h ? q.sc_hi : q.sc_lo, ok ? 16.f : 0.f, c);
+#pragma unroll
+    for (int t = 0; t < 4; t++) c[t] = __builtin_elementwise_fma(m[t], splat2(-kappa), c[t]);  // |.| <= 1953
+    S.mn = __builtin_bit_cast(uint4, h8{m[0].x, m[0].y, m[1].x, m[1].y, m[2].x, m[2].y, m[3].x, m[3].y});
+    S.rest = __builtin_bit_cast(uint4, h8{c[0].x, c[0].y, c[1].x, c[1].y, c[2].x, c[2].y, c[3].x, c[3].y});
+    reinterpret_cast<float*>(dl)[lane] = h == 0 ? dw : ok ? fmaf(-kappa, dw, dm) : dm;
+}
+
 // An infinite scale (an infinity in the block) makes every block dot of the
 // reference NaN: a zero sum times it, or main and min terms of one sign.  (The
 // quantizer does the same for the f16 image.)
@@ -350,8 +399,9 @@ __device__ __forceinline__ float finite_or_nan(float d) { return d - d == 0.0f ?
 
 // A super-block's sums I (and the min sums) of a 32 x 32 tile into the output.
 template <int DT>
-__device__ __forceinline__ void super_unit(const f16v& I, const Scales<DT>& S, const uint4& bs, float da, const float* dw,
+__device__ __forceinline__ void super_unit(f16v I, const Scales<DT>& S, const uint4& bs, float da, const float* dw,
                                            const float* dm, f16v& out) {
+    if constexpr (DT == XNQ_Q5K) I = mfma16(as_h8(S.rest), as_h8(bs), I);
     if constexpr (HT<DT>::kMinK) {
         const f16v I2 = mfma16(as_h8(S.mn), as_h8(bs), f16v{});
 #pragma unroll
@@ -537,10 +587,14 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
                 f16v I[TM];
 #pragma unroll
                 for (int j = 0; j < T::kCH; j++) {
+                    if constexpr (DT == XNQ_Q5K) {
+                        // (later, the two-tile form spills: 4096 -> 6144 m = 37 19.6 us against 16.8)
+                        if (j == 2) read_rest<DT>(S, dl, lane);
+                    }
                     h8 A[2];
                     Bytes by;
                     read_chunk<DT>(by, ws, lrow, j, g);
-                    expand<DT>(by, j, g, S.hd, A);
+                    expand<DT>(by, j, g, S, A);
 #pragma unroll
                     for (int i = 0; i < TM; i++) {
                         const int u = j * TM + i;
@@ -573,7 +627,7 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
                     h8 A[2];
                     Bytes by;
                     read_chunk<DT>(by, ws, lrow, j, g);
-                    expand<DT>(by, j, g, S.hd, A);
+                    expand<DT>(by, j, g, S, A);
 #pragma unroll
                     for (int i = 0; i < TM; i++) {
                         const int u = j * TM + i;
@@ -948,10 +1002,15 @@ __global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++) {
                     const int j = 4 * p + jj;
+                    if constexpr (DT == XNQ_Q5K) {
+                        // m = 512, 4096 -> 4096, us: here 53.7, after the products 57.3, before
+                        // them 59.3, with neither this nor the levels less 16 53.0
+                        if (j == 7) read_rest<DT>(S, dl, lane);
+                    }
                     h8 A[2];
                     Bytes by;
                     read_chunk<DT>(by, ws, lrow, j, g);
-                    expand<DT>(by, j, g, S.hd, A);
+                    expand<DT>(by, j, g, S, A);
 #pragma unroll
                     for (int i = 0; i < 2; i++) {
                         const uint4 b0 = *reinterpret_cast<const uint4*>(bs + i * 8192 + jj * 2048);
@@ -1156,7 +1215,7 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
         };
         read_chunk<DT>(by, ws, lrow, 0, g);
         read_b(0);
-        expand<DT>(by, 0, g, S.hd, A[0]);
+        expand<DT>(by, 0, g, S, A[0]);
         read_chunk<DT>(by, ws, lrow, 1, g);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -1165,7 +1224,7 @@ __global__ __launch_bounds__(1024) void h16_block_tile_kernel(WView w, AView a, 
             __builtin_amdgcn_sched_barrier(0);
             if (j < 3) {
                 read_b(j + 1);
-                expand<DT>(by, j + 1, g, S.hd, A[(j + 1) & 1]);
+                expand<DT>(by, j + 1, g, S, A[(j + 1) & 1]);
                 asm volatile("" : "+v"(A[(j + 1) & 1][0]), "+v"(A[(j + 1) & 1][1]));
                 if (j < 2) read_chunk<DT>(by, ws, lrow, j + 2, g);
             }
