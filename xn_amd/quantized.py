@@ -360,7 +360,8 @@ class QLinear:
     def forward(self, xs: torch.Tensor) -> torch.Tensor:
         """mod.rs:352-384: (..., k) -> (..., n), then + bias."""
         weight = self.weight
-        dims, shape = weight._shape, xs.shape
+        plain = type(weight) is QTensor  # not a subclass or another object with its own matmul_t
+        dims, shape = weight._shape if plain else weight.shape(), xs.shape
         if len(dims) != 2:
             raise XnqError(1, f"unexpected rank, expected: 2, got: {len(dims)} ({dims})")
         n, k = dims
@@ -368,11 +369,11 @@ class QLinear:
             raise XnqError(1, f"input tensor has only one dimension {tuple(shape)}")
         if shape[-1] != k:
             raise XnqError(1, f"input tensor {tuple(shape)} incompatible with {list(dims)}")
-        dev = weight.storage.device
+        dev = weight.storage.device if plain else weight.device
         dst = torch.empty(shape[:-1] + (n,), dtype=torch.float32, device=dev)
         xs = xs.contiguous()
         m = xs.numel() // k
-        if xs.dtype is torch.float32 and xs.device == dev:
+        if plain and xs.dtype is torch.float32 and xs.device == dev:
             weight._matmul_t(m, k, n, xs, dst)  # nothing of matmul_t's checks can fail
         else:
             weight.matmul_t((m, k, n), xs, dst)
