@@ -218,6 +218,12 @@ xnq_status xnq_qtensor_matmul_preq(const xnq_qtensor* qt, size_t m, size_t k, si
  * 3 = skinny int8-MFMA kernel (m <= 64).  Process wide. */
 xnq_status xnq_set_route(int route);
 
+/* The kernel that matmul_t takes for m rows and an n x k weight on the present
+ * route (testing): "matvec", "skinny", "prefill", "qmm", "h16_ksplit16",
+ * "h16_ksplit32", "h16_ksplit64", "h16_block_tile" or "h16_super_tile"; "" for
+ * a shape or dtype that it does not take.  Host only. */
+const char* xnq_matmul_t_kernel(uint32_t weight_dtype, size_t m, size_t n, size_t k);
+
 /* Dequantize into elem_count f32 values (QTensor::dequantize /
  * GgmlType::to_float, mod.rs:316-318). */
 xnq_status xnq_qtensor_dequantize(const xnq_qtensor* qt, float* dst_dev, size_t elem_count,

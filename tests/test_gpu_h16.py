@@ -30,7 +30,16 @@ def run(qt, x, m, k, n, dev):
     return dst.cpu().numpy()
 
 
-def check(orc, dev, dt, m, k, n, seed, wscale=0.02, xscale=1.0):
+def reaches(kernel, dt, m, k, n):
+    """The case is on the kernel that its test is about."""
+    from xn_amd.quantized import matmul_t_kernel
+
+    assert matmul_t_kernel(dt, m, n, k) == kernel, f"dt={dt} m={m} k={k} n={n}"
+
+
+def check(orc, dev, dt, m, k, n, seed, wscale=0.02, xscale=1.0, kernel=None):
+    if kernel:
+        reaches(kernel, dt, m, k, n)
     rng = np.random.default_rng(seed)
     blocks = orc.from_float(dt, (rng.normal(0, wscale, (n, k))).astype(np.float32))
     x = (rng.normal(0, xscale, (m, k))).astype(np.float32)
@@ -52,7 +61,35 @@ def test_block_types_ksplit(orc, dev, dt, m, k, n):
 @pytest.mark.parametrize("dt", BLOCK32)
 @pytest.mark.parametrize("m,k,n", [(9, 128, 31), (16, 640, 8200), (17, 1152, 33), (47, 4224, 67), (125, 2048, 100)])
 def test_block_types_16_rows(orc, dev, dt, m, k, n):
-    check(orc, dev, dt, m, k, n, 150 + dt + m)
+    check(orc, dev, dt, m, k, n, 150 + dt + m, kernel="h16_ksplit16")
+
+
+# 32-row tiles: one row tile (an even and a ragged one), K in whole and in cut stages
+@pytest.mark.parametrize("dt", BLOCK32)
+@pytest.mark.parametrize("m,k,n", [(64, 64, 4096), (33, 1088, 4065), (64, 512, 4096), (57, 2240, 4070)])
+def test_block_types_32_rows(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 170 + dt + m, kernel="h16_ksplit32")
+
+
+# 64-row tiles: both row tiles full, the second one ragged or missing, K in whole and in cut stages
+@pytest.mark.parametrize("dt", BLOCK32)
+@pytest.mark.parametrize("m,k,n", [(64, 1088, 8200), (41, 320, 8250), (70, 192, 8200), (96, 512, 8224)])
+def test_block_types_64_rows(orc, dev, dt, m, k, n):
+    check(orc, dev, dt, m, k, n, 190 + dt + m, kernel="h16_ksplit64")
+
+
+@pytest.mark.parametrize("dt", SUPER)
+@pytest.mark.parametrize("m,k,n,kernel", [(33, 512, 4065, "h16_ksplit32"), (64, 2304, 4096, "h16_ksplit32"),
+                                          (41, 512, 8250, "h16_ksplit64"), (70, 2304, 7900, "h16_ksplit64")])
+def test_super_types_row_tiles(orc, dev, dt, m, k, n, kernel):
+    check(orc, dev, dt, m, k, n, 350 + dt + m, kernel=kernel)
+
+
+# more 256 x 64 tiles than one round of workgroups
+@pytest.mark.parametrize("dt", BLOCK32 + SUPER)
+def test_second_round_of_tiles(orc, dev, dt):
+    kernel = "h16_super_tile" if dt in SUPER else "h16_block_tile"
+    check(orc, dev, dt, 1100, 256 if dt in SUPER else 64, 4608, 370 + dt, kernel=kernel)
 
 
 @pytest.mark.parametrize("dt", [Q4_0, Q8_0])
@@ -71,18 +108,18 @@ def test_super_types_ksplit(orc, dev, dt, m, k, n):
 @pytest.mark.parametrize("dt,m,k,n", [(dt, 640, 64, 4353) for dt in BLOCK32] + [(dt, 577, 2112, 4608) for dt in BLOCK32]
                          + [(dt, 600, 4160, 4352) for dt in (Q4_0, Q5_1, Q8_0)])
 def test_block_types_tile(orc, dev, dt, m, k, n):
-    check(orc, dev, dt, m, k, n, 400 + dt + m)
+    check(orc, dev, dt, m, k, n, 400 + dt + m, kernel="h16_block_tile")
 
 
 @pytest.mark.parametrize("dt", [Q4_0, Q8_0])
 def test_block_types_tile_odd_blocks(orc, dev, dt):
-    check(orc, dev, dt, 600, 1056, 4354, 500 + dt)
+    check(orc, dev, dt, 600, 1056, 4354, 500 + dt, kernel="h16_block_tile")
 
 
 @pytest.mark.parametrize("dt", SUPER)
 @pytest.mark.parametrize("m,k,n", [(512, 256, 4353), (449, 1280, 4352), (520, 4352, 4096)])
 def test_super_types_tile(orc, dev, dt, m, k, n):
-    check(orc, dev, dt, m, k, n, 600 + dt + m)
+    check(orc, dev, dt, m, k, n, 600 + dt + m, kernel="h16_super_tile")
 
 
 # block scales in the f16 subnormal range, on either side
@@ -130,6 +167,7 @@ def test_overflowing_block_sums(orc, dev, dt, m, n):
     x = np.random.default_rng(5850 + dt).normal(0, 1, (m, k)).astype(np.float32)
     x[3, 64:96], x[5, 128:160], x[7, 40], x[9, 288:] = 3000.0, -3000.0, 7e4, 2500.0
     x[11, 0:32], x[11, 96:128] = 3000.0, -3000.0
+    reaches({40: "h16_ksplit16", 600: "h16_block_tile"}.get(m, "h16_ksplit32" if n == 4096 else "h16_ksplit64"), dt, m, k, n)
     got, want = run_both(orc, dev, dt, m, k, n, x, 850 + dt)
     assert np.isinf(want[[3, 5, 7, 9]]).any(axis=1).all()
     check_nonfinite(got, want, m)
@@ -142,6 +180,8 @@ def test_overflowing_scale_in_a_cut_stage(orc, dev, dt, k, m, n):
     stages of four blocks: the blocks that fill the stage up add nothing."""
     x = np.random.default_rng(5870 + dt).normal(0, 1, (m, k)).astype(np.float32)
     x[3, -5], x[5, k - 32] = 1e9, -1e9
+    few = "h16_ksplit32" if dt in (Q4_0, Q8_0) else "h16_ksplit16"  # (scales of their own: no 16-row tiles of a cut stage)
+    reaches({40: few, 600: "h16_block_tile"}.get(m, "h16_ksplit32" if n == 4096 else "h16_ksplit64"), dt, m, k, n)
     got, want = run_both(orc, dev, dt, m, k, n, x, 870 + dt)
     if dt not in (Q4_1, Q5_1):  # (their infinite sum times m meets the infinite product)
         assert np.isinf(want[[3, 5]]).any(axis=1).all()
@@ -161,6 +201,8 @@ def test_nonfinite_rows(orc, dev, dt, m, n):
     x = rng.normal(0, 1, (m, k)).astype(np.float32)
     x[3, 7], x[5, 300], x[20, 40] = np.inf, np.nan, 1e9
     x[8] = 0.0
+    few = "h16_ksplit32" if dt in SUPER else "h16_ksplit16"
+    reaches(few if m == 40 else "h16_super_tile" if dt in SUPER else "h16_block_tile", dt, m, k, n)
     qt = upload(blocks, n, k, dt, dev)
     got = run(qt, x, m, k, n, dev)
     try:

@@ -68,15 +68,21 @@ def check(e):
     assert e[0] <= max(e[1], 2.0 ** -24), f"relative L2 error {e[0]:.3e}, matvec kernels {e[1]:.3e}"
 
 
-# 16-row, one and two 32-row K-split tiles; 256 x 64 tiles
-SHAPES = [(40, 1024, 96), (64, 1024, 4096), (64, 1024, 8224), (600, 2048, 4352)]
+# 16-row (K types: 32-row), 32- and 64-row K-split tiles; 256 x 64 tiles
+SHAPES = [(40, 1024, 96, "h16_ksplit16"), (64, 1024, 4096, "h16_ksplit32"), (64, 1024, 8224, "h16_ksplit64"),
+          (600, 2048, 4352, "tile")]
 
 
 @pytest.mark.parametrize("dt", TYPES)
-@pytest.mark.parametrize("m,k,n", SHAPES)
+@pytest.mark.parametrize("m,k,n,kernel", SHAPES)
 @pytest.mark.parametrize("offset", [0.0, 10.0])
-def test_no_larger_than_the_matvec(orc, dev, dt, m, k, n, offset):
+def test_no_larger_than_the_matvec(orc, dev, dt, m, k, n, kernel, offset):
     from xn_amd import GgmlDType, QTensor
+    from xn_amd.quantized import matmul_t_kernel
+
+    if dt in (Q2K, Q3K, Q5K):
+        kernel = {"h16_ksplit16": "h16_ksplit32", "tile": "h16_super_tile"}.get(kernel, kernel)
+    assert matmul_t_kernel(dt, m, n, k) == ("h16_block_tile" if kernel == "tile" else kernel)
 
     w = torch.empty((n, k), device=dev).normal_(0, 0.02, generator=torch.Generator(device=dev).manual_seed(40 + dt))
     blocks = np.frombuffer(QTensor.quantize_f32(w, dtype=GgmlDType(dt)).data(), np.uint8)

@@ -57,6 +57,7 @@ SIGNATURES = {
     "xnq_quantize_lhs": (c_int, [c_u32, c_size, c_size, c_void, c_void, c_void]),
     "xnq_qtensor_matmul_preq": (c_int, [c_void, c_size, c_size, c_size, c_void, c_size, c_void, c_void]),
     "xnq_set_route": (c_int, [c_int]),
+    "xnq_matmul_t_kernel": (ctypes.c_char_p, [c_u32, c_size, c_size, c_size]),
     "xnq_qtensor_dequantize": (c_int, [c_void, c_void, c_size, c_void]),
     "xnq_qtensor_raw_data": (c_int, [c_void, c_void, c_size, c_void]),
     "xnq_quantize_act_blocks": (c_int, [c_u32, c_size, c_size, c_void, c_void, c_void]),

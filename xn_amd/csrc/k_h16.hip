@@ -1287,37 +1287,54 @@ hipError_t launch_ksplit16(const WView& w, const AView& a, size_t m, float* y, h
     return hipGetLastError();
 }
 
+// The kernel of m rows by n columns: 16-, 32- or 64-row tiles with K split over the
+// wavefronts, or 256 x 64 tiles.
+enum class Form { kSplit16, kSplit32, kSplit64, kTile };
+
+// From the row images: 32-row tiles up to one workgroup per CU, then 64-row ones.
+Form rows_form(size_t m, size_t n) {
+    const size_t rts = (m + 31) / 32, n32 = (n + 31) / 32;
+    return rts == 1 || rts * n32 <= 256 ? Form::kSplit32 : Form::kSplit64;
+}
+
+template <int DT, bool DV>
+Form h16_form(size_t m, size_t n) {
+    const size_t n32 = (n + 31) / 32;
+    if (!HT<DT>::kK && DV) {
+        // 16-row tiles up to one workgroup per CU (two rounds of them against one of
+        // 32-row tiles: Q8_0 N = 4096 m = 64 19.3 / 14.7), and where 32 rows would be half
+        // padding.  Not where planed scales do not come with the stage (K % 128 != 0):
+        // loads of their own inside it lose (Q8_0 1056 -> 2048 m = 48 9.1 / 8.2)
+        if (m <= 16 || (m + 15) / 16 * n32 <= 256) return Form::kSplit16;
+    }
+    // 32-row tiles up to one workgroup per CU, then 64-row tiles (Q8_0, K = 4096, us, graph
+    // steps: N = 1024 m = 256 17 / 21, 512 31 / 25; N = 4096 m = 64 15 / 19, 128 25 / 21)
+    if (rows_form(m, n) == Form::kSplit32) return Form::kSplit32;
+    // A round of 256 x 64 tiles (one a CU) costs the same however few it holds; a round
+    // of 64-row K-split workgroups is the products of 32 tiles.  So the tile pays from
+    // so many K-split rounds, us, K = N = 4096, K-split / tile: Q2K m = 256 (2 rounds)
+    // 40 / 52, 320 (3) 59 / 52; Q5K 384 (3) 46 / 54, 448 (4) 58 / 55; Q3K 384 42 / 52,
+    // 512 (4) 54 / 52; Q8_0 512 (4) 66 / 67, 576 (5) 81 / 68; Q4_0 512 65 / 70, 576
+    // 79 / 70; Q4_1 512 140 / 141, 576 169 / 146; Q5_0 640 (5) 80 / 92, 768 (6) 97 / 93;
+    // Q5_1 640 133 / 135, 768 163 / 142; scales not staged (Q8_0, K = 4160) 640 88 / 103.
+    constexpr size_t kRounds = DT == XNQ_Q2K ? 2 : DT == XNQ_Q5K ? 3 : DT == XNQ_Q5_0 || DT == XNQ_Q5_1 || !DV ? 5 : 4;
+    const size_t tiles = ((m + 63) / 64) * ((n + 255) / 256), rounds = (tiles + 255) / 256;
+    return tiles <= rounds * kRounds * 32 ? Form::kSplit64 : Form::kTile;
+}
+
 template <int DT, bool DV>
 hipError_t launch_rows_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
-    const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
-    if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV, true>(w, a, m, y, s);
+    if (rows_form(m, w.n) == Form::kSplit32) return launch_ksplit<DT, 1, DV, true>(w, a, m, y, s);
     return launch_ksplit<DT, 2, DV, true>(w, a, m, y, s);
 }
 
 template <int DT, bool DV>
 hipError_t launch_h16_dt(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
-    const size_t rts = (m + 31) / 32, n32 = (w.n + 31) / 32;
-    if constexpr (!HT<DT>::kK && DV) {
-        // 16-row tiles up to one workgroup per CU (two rounds of them against one of
-        // 32-row tiles: Q8_0 N = 4096 m = 64 19.3 / 14.7), and where 32 rows would be half
-        // padding.  Not where planed scales do not come with the stage (K % 128 != 0):
-        // loads of their own inside it lose (Q8_0 1056 -> 2048 m = 48 9.1 / 8.2)
-        const size_t rt16 = (m + 15) / 16;
-        if (m <= 16 || rt16 * n32 <= 256) return launch_ksplit16<DT>(w, a, m, y, s);
-    }
-    // 32-row tiles up to one workgroup per CU, then 64-row tiles (Q8_0, K = 4096, us, graph
-    // steps: N = 1024 m = 256 17 / 21, 512 31 / 25; N = 4096 m = 64 15 / 19, 128 25 / 21)
-    if (rts == 1 || rts * n32 <= 256) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
-    // A round of 256 x 64 tiles (one a CU) costs the same however few it holds; a round
-    // of 64-row K-split workgroups is the products of 32 tiles.  So the tile pays from
-    // so many K-split rounds, us, K = N = 4096, K-split / tile: Q2K m = 256 (2 rounds)
-    // 40 / 52, 320 (3) 59 / 52; Q5K 384 (3) 46 / 52, 448 (4) 58 / 52; Q3K 384 42 / 52,
-    // 512 (4) 54 / 52; Q8_0 512 (4) 66 / 67, 576 (5) 81 / 68; Q4_0 512 65 / 70, 576
-    // 79 / 70; Q4_1 512 140 / 141, 576 169 / 146; Q5_0 640 (5) 80 / 92, 768 (6) 97 / 93;
-    // Q5_1 640 133 / 135, 768 163 / 142; scales not staged (Q8_0, K = 4160) 640 88 / 103.
-    constexpr size_t kRounds = DT == XNQ_Q2K ? 2 : DT == XNQ_Q5K ? 3 : DT == XNQ_Q5_0 || DT == XNQ_Q5_1 || !DV ? 5 : 4;
-    const size_t tiles = ((m + 63) / 64) * ((w.n + 255) / 256), rounds = (tiles + 255) / 256;
-    if (tiles <= rounds * kRounds * 32) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
+    const Form f = h16_form<DT, DV>(m, w.n);
+    if constexpr (!HT<DT>::kK && DV)
+        if (f == Form::kSplit16) return launch_ksplit16<DT>(w, a, m, y, s);
+    if (f == Form::kSplit32) return launch_ksplit<DT, 1, DV>(w, a, m, y, s);
+    if (f == Form::kSplit64) return launch_ksplit<DT, 2, DV>(w, a, m, y, s);
     const uint32_t m_tiles = (uint32_t)((m + 63) / 64), n_tiles = (w.n + 255) / 256, grid = (m_tiles * n_tiles + 7) / 8 * 8;
     if constexpr (HT<DT>::kK) {
         constexpr int kLds = TLay<DT>::kLds;
@@ -1339,34 +1356,44 @@ bool h16_supported(uint32_t dtype) {
     return dtype == XNQ_Q8_0 || dtype == XNQ_Q4_0 || is_raw_layout(dtype);
 }
 
-// launch_h16_dt or launch_rows_dt of the weight's type
-template <bool ROWS>
-static hipError_t launch_type(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
-#define XNQ_H16(DT, DV) (ROWS ? launch_rows_dt<DT, DV>(w, a, m, y, s) : launch_h16_dt<DT, DV>(w, a, m, y, s))
-    switch (w.dtype) {
-    case XNQ_Q8_0: return w.nb % 4 == 0 ? XNQ_H16(XNQ_Q8_0, true) : XNQ_H16(XNQ_Q8_0, false);
-    case XNQ_Q4_0: return w.nb % 4 == 0 ? XNQ_H16(XNQ_Q4_0, true) : XNQ_H16(XNQ_Q4_0, false);
-    case XNQ_Q4_1: return XNQ_H16(XNQ_Q4_1, true);
-    case XNQ_Q5_0: return XNQ_H16(XNQ_Q5_0, true);
-    case XNQ_Q5_1: return XNQ_H16(XNQ_Q5_1, true);
-    case XNQ_Q2K: return XNQ_H16(XNQ_Q2K, true);
-    case XNQ_Q3K: return XNQ_H16(XNQ_Q3K, true);
-    case XNQ_Q5K: return XNQ_H16(XNQ_Q5K, true);
+// f(type, whether the scales come with the stage) of a weight of type dt and nb blocks a row
+template <class F>
+static auto by_type(uint32_t dt, size_t nb, F f) {
+    using std::integral_constant;
+    switch (dt) {
+    case XNQ_Q8_0:
+        return nb % 4 == 0 ? f(integral_constant<int, XNQ_Q8_0>{}, std::true_type{})
+                           : f(integral_constant<int, XNQ_Q8_0>{}, std::false_type{});
+    case XNQ_Q4_0:
+        return nb % 4 == 0 ? f(integral_constant<int, XNQ_Q4_0>{}, std::true_type{})
+                           : f(integral_constant<int, XNQ_Q4_0>{}, std::false_type{});
+    case XNQ_Q4_1: return f(integral_constant<int, XNQ_Q4_1>{}, std::true_type{});
+    case XNQ_Q5_0: return f(integral_constant<int, XNQ_Q5_0>{}, std::true_type{});
+    case XNQ_Q5_1: return f(integral_constant<int, XNQ_Q5_1>{}, std::true_type{});
+    case XNQ_Q2K: return f(integral_constant<int, XNQ_Q2K>{}, std::true_type{});
+    case XNQ_Q3K: return f(integral_constant<int, XNQ_Q3K>{}, std::true_type{});
+    default: return f(integral_constant<int, XNQ_Q5K>{}, std::true_type{});  // Q5K (h16_supported types only)
     }
-#undef XNQ_H16
-    return hipErrorNotSupported;
+}
+
+const char* h16_kernel(uint32_t dtype, size_t m, size_t n, size_t k) {
+    const Form f = by_type(dtype, k / 32, [&](auto dt, auto dv) { return h16_form<dt.value, dv.value>(m, n); });
+    if (f == Form::kTile) return is_kquant(dtype) ? "h16_super_tile" : "h16_block_tile";
+    return f == Form::kSplit16 ? "h16_ksplit16" : f == Form::kSplit32 ? "h16_ksplit32" : "h16_ksplit64";
 }
 
 hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (!a.h16 || (size_t)a.H.rts * 32 < m || a.k != w.k) return hipErrorInvalidValue;
-    return launch_type<false>(w, a, m, y, s);
+    if (!h16_supported(w.dtype)) return hipErrorNotSupported;
+    return by_type(w.dtype, w.nb, [&](auto dt, auto dv) { return launch_h16_dt<dt.value, dv.value>(w, a, m, y, s); });
 }
 
 hipError_t launch_h16_rows(const WView& w, const AView& a, size_t m, float* y, hipStream_t s) {
     if (m == 0 || w.n == 0) return hipSuccess;
     if (a.m < m || a.k != w.k) return hipErrorInvalidValue;
-    return launch_type<true>(w, a, m, y, s);
+    if (!h16_supported(w.dtype)) return hipErrorNotSupported;
+    return by_type(w.dtype, w.nb, [&](auto dt, auto dv) { return launch_rows_dt<dt.value, dv.value>(w, a, m, y, s); });
 }
 
 }  // namespace xnq

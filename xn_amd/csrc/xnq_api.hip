@@ -534,6 +534,17 @@ static Route pick_route(uint32_t dtype, size_t m, size_t n, size_t k, int forced
     return kMatvec;
 }
 
+const char* xnq_matmul_t_kernel(uint32_t weight_dtype, size_t m, size_t n, size_t k) {
+    if (!device_dtype(weight_dtype) || m == 0 || n == 0 || k == 0 || k % block_size(weight_dtype)) return "";
+    switch (pick_route(weight_dtype, m, n, k, g_route.load())) {
+    case kH16: return h16_kernel(weight_dtype, m, n, k);
+    case kMfma:
+        return prefill_supported(weight_dtype, m, n, k) ? "prefill" : mfma_supported(weight_dtype, m, n, k) ? "qmm" : "";
+    case kSkinny: return skinny_supported(weight_dtype, m, n, k) ? "skinny" : "";
+    default: return "matvec";
+    }
+}
+
 // Split-K partial sums sit after the activation image in the workspace.
 static size_t partial_offset(uint32_t dtype, size_t m, size_t k, int forced) {
     return (act_layout(dtype, m, k, forced).bytes + kAlign - 1) / kAlign * kAlign;

@@ -319,6 +319,7 @@ hipError_t launch_prefill(const WView& w, const AView& a, size_t m, uint32_t spl
 
 // k_h16.hip: the f16 matrix-core kernels of the other weight types
 bool h16_supported(uint32_t dtype);
+const char* h16_kernel(uint32_t dtype, size_t m, size_t n, size_t k);  // the one launch_h16 takes
 hipError_t launch_h16(const WView& w, const AView& a, size_t m, float* y, hipStream_t s);
 // the same from the row images alone
 hipError_t launch_h16_rows(const WView& w, const AView& a, size_t m, float* y, hipStream_t s);

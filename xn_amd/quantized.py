@@ -532,6 +532,11 @@ def set_route(route: int) -> None:
     check(_lib.load().xnq_set_route(int(route)))
 
 
+def matmul_t_kernel(dtype: GgmlDType, m: int, n: int, k: int) -> str:
+    """Name of the kernel matmul_t takes for m rows and an n x k weight (see xnq.h)."""
+    return _lib.load().xnq_matmul_t_kernel(int(dtype), m, n, k).decode()
+
+
 def lhs_workspace(dtype: GgmlDType, m: int, k: int, device) -> torch.Tensor:
     nbytes = _lib.load().xnq_lhs_workspace_size(int(dtype), m, k)
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=device)
