@@ -114,3 +114,23 @@ def test_workspace_of_the_row_images(orc, dev, dt):
     check(_lib.load().xnq_matmul_t_group(hs, 2, m, k, xt.data_ptr(), ds, ws.data_ptr(), ws.numel(),
                                          torch.cuda.current_stream().cuda_stream))
     assert close(ys[0], want[0]) and close(ys[1], want[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [Q8_0, Q5_1, Q3K, Q5K])
+@pytest.mark.parametrize("n", [96, 65 * 256])  # (a K split and the tile of the f16 image, where it is aligned)
+def test_workspace_off_its_alignment(orc, dev, dt, n):
+    """Workspace, rows and output at addresses of 4-byte alignment."""
+    from xn_amd import GgmlDType, QTensor
+
+    m, k = 130, 512
+    rng = np.random.default_rng(960 + dt)
+    blocks = orc.from_float(dt, rng.normal(0, 0.02, (n, k)).astype(np.float32))
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    qt = QTensor.from_gguf_bytes(blocks, (n, k), GgmlDType(dt), dev)
+    ws = torch.zeros(qt.matmul_t_workspace_size(m) + 260, dtype=torch.uint8, device=dev)
+    xt, y = torch.empty(m * k + 1, device=dev), torch.full((m * n + 1,), float("nan"), device=dev)
+    xt[1:] = torch.from_numpy(x).to(dev).reshape(-1)
+    qt.matmul_t_ws((m, k, n), xt[1:], ws[4:], y[1:])
+    got, want = y[1:].view(m, n).cpu().numpy().astype(np.float64), orc.matmul(dt, x, blocks, n).astype(np.float64)
+    assert np.linalg.norm(got - want) < 2e-6 * np.linalg.norm(want)

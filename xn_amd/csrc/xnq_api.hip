@@ -656,6 +656,18 @@ size_t xnq_qtensor_matmul_t_workspace_size(const xnq_qtensor* qt, size_t m) {
     return matmul_t_workspace_size_impl(qt, m, g_route.load());
 }
 
+// The route of a call on the caller's workspace.  One that holds the row images but
+// not the f16 image (all that these types took with the matvec kernels) serves as in
+// matmul_preq, and so does one that is not 16-byte aligned: the f16 image's tiles are
+// fetched with 16-byte LDS DMA, the row images with plain loads, as the matvec
+// kernels read them.
+static int ws_route(uint32_t weight_dtype, size_t m, size_t k, int forced, const void* workspace_dev,
+                    size_t workspace_bytes) {
+    const ALayout L = act_layout(weight_dtype, m, k, forced);
+    const bool fits = workspace_bytes >= L.bytes && (uintptr_t)workspace_dev % 16 == 0;
+    return !L.h16 || fits ? forced : two_call(weight_dtype, forced);
+}
+
 static xnq_status matmul_t_ws_impl(const xnq_qtensor* qt, size_t m, size_t k, size_t n, const float* lhs_dev,
                                    void* workspace_dev, size_t workspace_bytes, float* dst_dev, void* stream,
                                    int forced) {
@@ -676,13 +688,8 @@ static xnq_status matmul_t_ws_impl(const xnq_qtensor* qt, size_t m, size_t k, si
         if (e != hipSuccess) return hip_fail(e, "matvec kernel");
         return XNQ_OK;
     }
-    size_t need = act_layout(qt->L.dtype, m, k, forced).bytes;
-    if (workspace_bytes < need) {
-        // one that holds the row images but not the f16 image (all that these types
-        // took with the matvec kernels) serves as in matmul_preq
-        forced = two_call(qt->L.dtype, forced);
-        need = act_layout(qt->L.dtype, m, k, forced).bytes;
-    }
+    forced = ws_route(qt->L.dtype, m, k, forced, workspace_dev, workspace_bytes);
+    const size_t need = act_layout(qt->L.dtype, m, k, forced).bytes;
     if (!workspace_dev || workspace_bytes < need)
         return fail(XNQ_ERR_INVALID, "workspace of %zu bytes is smaller than the %zu the activation needs",
                     workspace_bytes, need);
@@ -935,9 +942,10 @@ static xnq_status silu_gate_impl(const xnq_qtensor* gate, const xnq_qtensor* up,
     if (shared_quantize(pair, 2, m, forced)) {
         DeviceGuard g(gate->device);
         if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
-        st = quantize_lhs_impl(gate->L.dtype, m, k, lhs_dev, workspace_dev, stream, forced);
-        if (!st) st = matmul_preq_impl(gate, m, k, n, workspace_dev, off, dst_dev, stream, forced);
-        if (!st) st = matmul_preq_impl(up, m, k, n, workspace_dev, off, u, stream, forced);
+        const int route = ws_route(gate->L.dtype, m, k, forced, workspace_dev, off);
+        st = quantize_lhs_impl(gate->L.dtype, m, k, lhs_dev, workspace_dev, stream, route);
+        if (!st) st = matmul_preq_impl(gate, m, k, n, workspace_dev, off, dst_dev, stream, route);
+        if (!st) st = matmul_preq_impl(up, m, k, n, workspace_dev, off, u, stream, route);
     } else {
         st = matmul_t_ws_impl(gate, m, k, n, lhs_dev, workspace_dev, off, dst_dev, stream, forced);
         if (!st) st = matmul_t_ws_impl(up, m, k, n, lhs_dev, workspace_dev, off, u, stream, forced);
@@ -1062,12 +1070,8 @@ xnq_status xnq_matmul_t_group(const xnq_qtensor* const* qts, size_t count, size_
                                 forced);
     if (shared_quantize(qts, count, m, forced)) {
         // one activation image for every weight, then one matmul each
-        int route = forced;
-        size_t need = act_layout(qts[0]->L.dtype, m, k, route).bytes;
-        if (workspace_bytes < need) {  // as in matmul_t_ws
-            route = two_call(qts[0]->L.dtype, forced);
-            need = act_layout(qts[0]->L.dtype, m, k, route).bytes;
-        }
+        const int route = ws_route(qts[0]->L.dtype, m, k, forced, workspace_dev, workspace_bytes);
+        const size_t need = act_layout(qts[0]->L.dtype, m, k, route).bytes;
         if (!workspace_dev || workspace_bytes < need)
             return fail(XNQ_ERR_INVALID, "workspace of %zu bytes is smaller than the %zu the activation needs",
                         workspace_bytes, need);
