@@ -416,10 +416,15 @@ __device__ __forceinline__ void super_unit(f16v I, const Scales<DT>& S, const ui
 // Few rows, or few tiles: a workgroup owns 32 weight columns and 32 TM rows,
 // and its eight wavefronts split K, so that a weight of a few thousand columns
 // still puts two wavefronts on every SIMD.  Each wavefront streams its share of
-// the weights through its own LDS ring (LDS DMA in whole cache lines, two
-// stages ahead) and its share of the activation image straight into registers
-// (a stage ahead); there is no barrier until the eight partial tiles are added
-// through LDS.
+// the weights through its own LDS ring (LDS DMA in whole cache lines) and its
+// share of the activation image straight into registers (a stage ahead); there
+// is no barrier until the eight partial tiles are added through LDS.
+//
+// The ring holds two stages beyond the present one, but the DMA does not run that
+// far ahead: a stage's is issued after the activation loads of the next one, and the
+// waits that the compiler places for those loads know nothing of it and so drain it
+// too, for the most part within the stage it was issued in (with one row tile Q5K's
+// all of it).  A stage therefore still meets the latency of its weights in part.
 // ---------------------------------------------------------------------------
 // The eight wavefronts' partials of four outputs, added in 64 bits: one rounding
 // for the eight, which pays for those of the longer chains over a wavefront's
