@@ -2,7 +2,7 @@
 they take, at the edges of their tiles (16, 32 and 64 rows, 32 and 256 columns),
 of their K stages (128 and 256, with the remainders of K), and of the rule
 that chooses between them; tiny (f16 subnormal) scales; infinities and NaN in
-the activations against the matvec kernels; the slabs of matmul_t_noalloc.
+the activations (and Q3_K's scales) against the matvec kernels; the slabs of matmul_t_noalloc.
 
 The kernels' block sums are exact integers and their sums over K are 32-bit,
 so the outputs are held to 32-bit sums of K / 32 terms: relative L2 2e-6
@@ -216,6 +216,36 @@ def test_nonfinite_rows(orc, dev, dt, m, n):
     ok = np.isfinite(want).all(axis=1)
     err = np.linalg.norm(got[ok].astype(np.float64) - want[ok]) / np.linalg.norm(want[ok].astype(np.float64))
     assert err < 2e-6
+
+
+@pytest.mark.parametrize("m,n,kernel", [(40, 64, "h16_ksplit32"), (64, 8224, "h16_ksplit64"), (512, 4384, "h16_super_tile")])
+def test_infinite_q3k_block_scales(orc, dev, m, n, kernel):
+    """The reference multiplies eight sums of a super-block by its scale; an infinite one
+    leaves NaN unless all eight are of one sign (1 output in 128), as on the matvec kernels."""
+    from xn_amd.quantized import set_route
+
+    k = 512
+    reaches(kernel, Q3K, m, k, n)
+    rng = np.random.default_rng(940)
+    blocks = np.frombuffer(bytes(orc.from_float(Q3K, rng.normal(0, 0.02, (n, k)).astype(np.float32))), np.uint8).copy()
+    cols = {3: np.inf, 31: -np.inf, 33: np.nan, n - 1: np.inf}
+    for c, v in cols.items():
+        blocks.reshape(n, k // 256, 110)[c, c % 2, 108:] = np.array([v], np.float16).view(np.uint8)
+    x = rng.normal(0, 1, (m, k)).astype(np.float32)
+    qt, xt = upload(blocks, n, k, Q3K, dev), torch.from_numpy(x).to(dev)
+    outs = [torch.empty((m, n), device=dev) for _ in range(3)]
+    qt.matmul_t((m, k, n), xt, outs[0])
+    qt.matmul_t_split((m, k, n), xt, outs[1])
+    try:
+        set_route(1)
+        qt.matmul_t((m, k, n), xt, outs[2])
+    finally:
+        set_route(0)
+    got, rows, want = (y.cpu().numpy() for y in outs)
+    hit = np.isin(np.arange(n), list(cols))
+    assert np.isnan(want[:, hit]).mean() > 0.9
+    for y in (got, rows):
+        assert np.isnan(y[:, hit]).all() and np.isfinite(y[:, ~hit]).all()
 
 
 @pytest.mark.parametrize("dt", [Q8_0, Q5K])

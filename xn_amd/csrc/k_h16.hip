@@ -265,6 +265,12 @@ __device__ __forceinline__ f16v mfma8(uint2 a, uint2 b) {
 }
 __device__ __forceinline__ h8 as_h8(uint4 v) { return __builtin_bit_cast(h8, v); }
 
+// An infinite activation scale (an infinity in the block) makes every block dot of the
+// reference NaN: a zero sum times it, or main and min terms of one sign.  (The
+// quantizer does the same for the f16 image.)  So does an infinite weight scale of Q3K,
+// whose reference multiplies eight sums of either sign by it (k_quants.rs:1071-1152).
+__device__ __forceinline__ float finite_or_nan(float d) { return fmaf(d, 0.0f, d); }
+
 // Reads a stage's scales from its slot; K types also leave d_w and dmin by
 // column at dl (a wavefront's own LDS: its operations stay in order).
 template <int DT, bool DV>
@@ -289,7 +295,9 @@ __device__ __forceinline__ void read_scales(Scales<DT>& S, const WView& w, const
             const float dw = f16_bits_to_f32(dd & 0xffffu);
             S.bias = dw - dw == 0.f ? -272.f : -256.f;
         } else {
-            reinterpret_cast<float*>(dl)[lane] = f16_bits_to_f32(h ? dd >> 16 : dd & 0xffffu);  // [dw 32][dmin 32]
+            // [dw 32][dmin 32] (Q3K: d_w twice)
+            const float d = f16_bits_to_f32(T::kMinK && h ? dd >> 16 : dd & 0xffffu);
+            reinterpret_cast<float*>(dl)[lane] = DT == XNQ_Q3K ? finite_or_nan(d) : d;
         }
         if constexpr (DT == XNQ_Q2K) {
             // mins of sub-blocks (16 elements each) 8h .. 8h + 7
@@ -391,11 +399,6 @@ __device__ __forceinline__ void read_rest(Scales<DT>& S, uint8_t* dl, uint32_t l
     S.rest = __builtin_bit_cast(uint4, h8{c[0].x, c[0].y, c[1].x, c[1].y, c[2].x, c[2].y, c[3].x, c[3].y});
     reinterpret_cast<float*>(dl)[lane] = h == 0 ? dw : ok ? fmaf(-kappa, dw, dm) : dm;
 }
-
-// An infinite scale (an infinity in the block) makes every block dot of the
-// reference NaN: a zero sum times it, or main and min terms of one sign.  (The
-// quantizer does the same for the f16 image.)
-__device__ __forceinline__ float finite_or_nan(float d) { return d - d == 0.0f ? d : d - d; }
 
 // A super-block's sums I (and the min sums) of a 32 x 32 tile into the output.
 template <int DT>
