@@ -119,7 +119,8 @@ xnq_status xnq_qtensor_matmul_t(const xnq_qtensor* qt, size_t m, size_t k, size_
  * to 6144 x 4096 elements: the row quantized in LDS by the matvec kernel;
  * workspace_dev may then be NULL).  A smaller one that still holds
  * xnq_lhs_workspace_size(dtype, m, k) bytes also serves, on slower kernels
- * where the f16 MFMA kernels would use the rest.  Same contract as xnq_qtensor_matmul_t
+ * where the f16 MFMA kernels would use the rest; so does, for the dtypes of those,
+ * one that is not 16-byte aligned.  Same contract as xnq_qtensor_matmul_t
  * (QTensor::matmul_t, mod.rs:334-339; k_quants::matmul, k_quants.rs:1996-2011). */
 size_t xnq_qtensor_matmul_t_workspace_size(const xnq_qtensor* qt, size_t m);
 xnq_status xnq_qtensor_matmul_t_ws(const xnq_qtensor* qt, size_t m, size_t k, size_t n,

@@ -6,8 +6,8 @@ the route boundaries instead: m from 1 to 700, so every route and both
 sides of each crossover are hit (matvec, the wavefront-split and split-K
 skinny kernels, the prefill kernel, the tiled kernel and its half-empty-tail
 instance); n ragged against every tile width; k any whole number of blocks
-(super-blocks for the K-quants); the six padded-block dtypes, which run on
-the matvec kernels at every m, are drawn the same way.  Reference semantics: k_quants::matmul
+(super-blocks for the K-quants); the six padded-block dtypes (matvec up to
+8 rows, f16 matrix-core kernels above) are drawn the same way.  Reference semantics: k_quants::matmul
 (k_quants.rs:1996-2011) over each dtype's vec_dot; the oracle's matmul is
 the check, to the f32 bar (1e-3 relative L2, 2e-3 max relative per row).
 """

@@ -1075,12 +1075,15 @@ __global__ __launch_bounds__(kThreads) void h16_super_tile_kernel(WView w, AView
 // ---------------------------------------------------------------------------
 // The 32-element types at prefill sizes.  A unit (32 x 32 x 32) is 3 MFMAs, 20
 // vector operations to fold it, and 20 to 24 (Q5: 40) to expand its weights: the
-// vector units bound it (1.8 ns an operation beside MFMAs, 14 ns an MFMA), and
-// two wavefronts per SIMD left them idle while both waited (LDS 33 % of the
-// time).  So sixteen wavefronts, four per SIMD, with one 32 x 32 tile each (a
-// column group's weights are fetched once for its two wavefronts and expanded
-// by both): M = 512, 4096 -> 14336, one box, us a step with the quantizer, 8
-// wavefronts of 32 x 64 on 16 x 16 tiles / this: Q4_0 162 / 148, Q8_0 161 / 145.
+// vector units bound it (issuing for 70 % of the cycles of Q4_0's dispatch, MFMAs
+// for 30 %), and two wavefronts per SIMD left them idle while both waited for LDS.
+// So sixteen wavefronts, four per SIMD, with one 32 x 32 tile each (a column
+// group's weights are fetched once for its two wavefronts and expanded by both):
+// M = 512, 4096 -> 14336, graph steps with the quantizer, weights rotated over
+// 600 MB, us, 8 wavefronts of 32 x 64 on 16 x 16 tiles / this: Q4_0 153 / 136, Q8_0
+// 158 / 137, Q5_0 190 / 176.  Q4_1 and Q5_1, whose min products do not fit the
+// registers beside the rest, lose: 259 / 348 and 236 / 282 (part of it, Q4_1 23,
+// to the shorter chains of sums below).
 // Three slots of LDS where they fit, fetched two steps ahead, else two.
 // ---------------------------------------------------------------------------
 template <int DT>
