@@ -477,7 +477,10 @@ __global__ __launch_bounds__(kThreads) void h16_ksplit_kernel(WView w, AView a, 
                                                               uint32_t n_tiles, float* __restrict__ y) {
     using T = HT<DT>;
     constexpr int kU = T::kCH * TM;       // (chunk, tile) units of a stage
-    constexpr int kPD = kU < 8 ? kU : 8;  // units whose operand B is in flight
+    // Units whose operand B is in flight: 8, but half of that for Q4_1 and Q5_1 on two row tiles,
+    // whose min products' operands are registers more: with 8 they spilled 72 and 52, with 4 9
+    // and 5 (8192 -> 6144 m = 64, graph steps, us, 60.6 / 33.0 and 46.6 / 32.0).
+    constexpr int kPD = T::kMin32 && TM == 2 && !ROWS ? 4 : kU < 8 ? kU : 8;
     constexpr int kSlots = 3, kWaveLds = kSlots * T::kSlot + T::kDl;
     constexpr int kRed = kWaves * TM * 4 * 64 * 16;
     constexpr int kLds = kWaves * kWaveLds > kRed ? kWaves * kWaveLds : kRed;
@@ -1326,8 +1329,11 @@ Form h16_form(size_t m, size_t n) {
     // so many K-split rounds, us, K = N = 4096, K-split / tile: Q2K m = 256 (2 rounds)
     // 40 / 52, 320 (3) 59 / 52; Q5K 384 (3) 46 / 54, 448 (4) 58 / 55; Q3K 384 42 / 52,
     // 512 (4) 54 / 52; Q8_0 512 (4) 66 / 67, 576 (5) 81 / 68; Q4_0 512 65 / 70, 576
-    // 79 / 70; Q4_1 512 140 / 141, 576 169 / 146; Q5_0 640 (5) 80 / 92, 768 (6) 97 / 93;
-    // Q5_1 640 133 / 135, 768 163 / 142; scales not staged (Q8_0, K = 4160) 640 88 / 103.
+    // 79 / 70; Q5_0 640 (5) 80 / 92, 768 (6) 97 / 93; scales not staged (Q8_0, K = 4160) 640
+    // 88 / 103.  Q4_1's and Q5_1's lines were drawn when their 64-row K-split kernels spilled (512
+    // 140 / 141, 640 133 / 135); these are the faster ones now up to 8 rounds (Q4_1 576 93 / 146,
+    // 1024 157 / 174; Q5_1 704 103 / 139, 1024 149 / 152), except Q5_1 over a short K (K = 1024
+    // 768 43 / 43, 1024 56 / 47), and the lines have not been drawn anew.
     constexpr size_t kRounds = DT == XNQ_Q2K ? 2 : DT == XNQ_Q5K ? 3 : DT == XNQ_Q5_0 || DT == XNQ_Q5_1 || !DV ? 5 : 4;
     const size_t tiles = ((m + 63) / 64) * ((n + 255) / 256), rounds = (tiles + 255) / 256;
     return tiles <= rounds * kRounds * 32 ? Form::kSplit64 : Form::kTile;
